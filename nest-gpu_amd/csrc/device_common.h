@@ -9,8 +9,71 @@
 #include "common.h"
 #include "kernels.h"
 #include "philox.h"
+#include "stepfactor.h"
 
 namespace ngpu {
+
+// ---------------------------------------------------------------------------
+// Division by a parameter d through its reciprocal R = 1/d in double:
+// RN32(x * R).  R and the product are within 2^-51 (relative) of the exact
+// quotient x/d, and the quotient of two floats is never within 2^-49 of a
+// midpoint between normal floats, so the result is the IEEE quotient, zeros,
+// infinities and NaN included.  A subnormal quotient can be an exact tie,
+// which the product may miss: a nonzero one is noted in `tiny` (the smallest
+// of (bits << 1) - 1; zeros wrap to the largest value).  Three instructions
+// and a half of bookkeeping, against three and four compares of the
+// single-precision form with a remainder correction it replaces.
+__device__ inline float div_recip(float x, double r, unsigned int& tiny) {
+  const float q = (float)((double)x * r);
+  tiny = min(tiny, (__float_as_uint(q) << 1) - 1u);
+  return q;
+}
+__device__ inline bool tiny_noted(unsigned int tiny) { return tiny < 0xffffffu; }
+
+// 1/d in double (d a normal float): the hardware estimate, good to ~2^-23,
+// and two Newton steps (relative error below 2^-52)
+__device__ inline double recip_double(float d) {
+  const double D = (double)d;
+  double r = __builtin_amdgcn_rcp(D);
+  r = fma(fma(-D, r, 1.0), r, r);
+  return fma(fma(-D, r, 1.0), r, r);
+}
+
+// the same of a wave-uniform d, in scalar registers
+__device__ inline double recip_uniform(float d) {
+  const long long b = __double_as_longlong(recip_double(d));
+  const unsigned int lo = __builtin_amdgcn_readfirstlane((int)b);
+  const unsigned int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// err^-1/5 (five) or err^-1/4 (not five), the floats of pow_m02 / pow_m025.
+// From the hardware's single-precision log2 and exp2 (relative error e of
+// y ~ x^-1/n below 2^-20) one correction in double with the terms to e^2 of
+// (1 - d)^(-1/n), d = 1 - x y^n, leaves an error below 2^-50: correctly
+// rounded for every float in [kPowLo, kPowHi] (exhaustive comparison with
+// pow_m02 / pow_m025 on the device), where those take three Newton steps
+// from a quadratic start, a binade split and a division of the exponent.
+// Outside the range, where a lane needs the value, those are called.
+constexpr float kPowLo = 0x1p-40f, kPowHi = 0x1p100f;
+__device__ inline float pow_step_fast(float x, bool five) {
+  const float y0 = __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(x) * (five ? -0.2f : -0.25f));
+  const double y = (double)y0, X = (double)x;
+  const double y2 = y * y;
+  const double y4 = y2 * y2;
+  const double yn = five ? y4 * y : y4;
+  const double d = fma(-X, yn, 1.0);
+  const double c = d * fma(d, five ? 0.12 : 0.15625, five ? 0.2 : 0.25);
+  return (float)fma(y, c, y);
+}
+__device__ inline float pow_step_dev(float x, bool five, bool need) {
+  float r = pow_step_fast(x, five);
+  if (__builtin_expect(__any(need && !(x >= kPowLo && x <= kPowHi)), 0)) {
+    const float s = five ? pow_m02(x) : pow_m025(x);
+    r = (x >= kPowLo && x <= kPowHi) ? r : s;
+  }
+  return r;
+}
 
 // ---------------------------------------------------------------------------
 // Spike emission: append to this step's spike list and do the per-node

@@ -1758,6 +1758,7 @@ int Engine::Calibrate() {
   if (const char* env = getenv("NGPU_FUSED_DELIVER")) fused_deliver_env_ = atoi(env) != 0;
   if (const char* env = getenv("NGPU_LAG_D0")) lag_d0_mode_ = atoi(env) == 1 ? 1 : 0;
   if (const char* env = getenv("NGPU_RK5_HOT_LANES")) rk5_hot_lanes_ = std::min(64, std::max(1, atoi(env)));
+  if (const char* env = getenv("NGPU_RK5_CHAIN_WAVES")) rk5_chain_waves_ = std::max(0, atoi(env));
   if (const char* env = getenv("NGPU_RK5_LEARNED_CAP")) rk5_learned_cap_ = std::max(0, atoi(env));
   if (const char* env = getenv("NGPU_RK5_DEFER")) {
     rk5_defer_cap_ = std::max(0, atoi(env));
@@ -2021,6 +2022,7 @@ RK5Args Engine::rk5_args(Group& gr, const StepCtx& sc, const SpikeList& sl, cons
     a.hot_margin = rk5_hot_margin_;
     a.hot_only = rk5_hot_only_ ? 1 : 0;
     a.hot_lanes = rk5_hot_lanes_;
+    a.chain_waves = rk5_chain_waves_;
   }
   if (g->lag.p) {
     a.lag = g->lag.p;

@@ -16,6 +16,7 @@
 #include "device_common.h"
 #include "kernels.h"
 #include "predictor_device.h"
+#include "rk5_chain.h"
 #include "rk5_models.h"
 #include "stepfactor.h"
 
@@ -49,6 +50,34 @@ constexpr int kMaxAttempts = 100000;
 }  // namespace ck
 using ck::kMaxAttempts;
 
+// The tableau as literals, and as vector registers: a v_fma_f32 takes no
+// literal, so literals sit in scalar registers, and a kernel that holds more
+// constants, parameters and pointers than its ~100 scalar registers reads
+// them back from vector lanes (v_readlane) in every iteration.
+struct CkConst {
+  static constexpr float a21 = ck::a21, a31 = ck::a31, a32 = ck::a32, a41 = ck::a41;
+  static constexpr float a42 = ck::a42, a43 = ck::a43, a51 = ck::a51, a52 = ck::a52;
+  static constexpr float a53 = ck::a53, a54 = ck::a54, a61 = ck::a61, a62 = ck::a62;
+  static constexpr float a63 = ck::a63, a64 = ck::a64, a65 = ck::a65, b1 = ck::b1;
+  static constexpr float b3 = ck::b3, b4 = ck::b4, b6 = ck::b6, e1 = ck::e1;
+  static constexpr float e3 = ck::e3, e4 = ck::e4, e5 = ck::e5, e6 = ck::e6;
+};
+struct CkRegs {
+  float a21 = ck::a21, a31 = ck::a31, a32 = ck::a32, a41 = ck::a41;
+  float a42 = ck::a42, a43 = ck::a43, a51 = ck::a51, a52 = ck::a52;
+  float a53 = ck::a53, a54 = ck::a54, a61 = ck::a61, a62 = ck::a62;
+  float a63 = ck::a63, a64 = ck::a64, a65 = ck::a65, b1 = ck::b1;
+  float b3 = ck::b3, b4 = ck::b4, b6 = ck::b6, e1 = ck::e1;
+  float e3 = ck::e3, e4 = ck::e4, e5 = ck::e5, e6 = ck::e6;
+  // values the compiler cannot see through, so they stay where they are
+  __device__ inline void hold() {
+    asm volatile("" : "+v"(a21), "+v"(a31), "+v"(a32), "+v"(a41), "+v"(a42), "+v"(a43));
+    asm volatile("" : "+v"(a51), "+v"(a52), "+v"(a53), "+v"(a54), "+v"(a61), "+v"(a62));
+    asm volatile("" : "+v"(a63), "+v"(a64), "+v"(a65), "+v"(b1), "+v"(b3), "+v"(b4));
+    asm volatile("" : "+v"(b6), "+v"(e1), "+v"(e3), "+v"(e4), "+v"(e5), "+v"(e6));
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Neuron models (right-hand sides and post-step updates).
 // Parameter and variable indices follow the reference's name tables.  Each
@@ -60,28 +89,18 @@ using ck::kMaxAttempts;
 // Every division of a right-hand side is by a parameter (M::divisor(j)).
 // dv.div(x, p, j) returns x / p[j].  DivIEEE divides.  DivFast, for
 // populations whose divisor parameters are uniform with a usable
-// reciprocal, multiplies by r[j] = RN(1/p[j]) and applies Markstein's
-// remainder correction, 3 multiply/fma giving the IEEE quotient for
-// dividends with magnitude in [2^-64, 2^64) and +0 (div_rn); any other
-// dividend (tiny, huge, inf, NaN, -0) only sets `bad`, and rhs() evaluates
-// the whole right-hand side again with DivIEEE when a lane of the wave has
-// it set: one wave-uniform branch, normally not taken, per evaluation
-// instead of a branch per division.  A negated dividend -x/d is written
-// -(x/d) (the same IEEE result) so that x = +0 stays on the fast path.
+// reciprocal, multiplies by the double reciprocal (div_recip: the IEEE
+// quotient of every dividend, but where the quotient is subnormal, which is
+// noted), and rhs() evaluates the whole right-hand side again with DivIEEE
+// when a lane of the wave has a nonzero subnormal quotient: one wave-uniform
+// branch, normally not taken, per evaluation.
 struct DivIEEE {
   __device__ inline float div(float x, const float* p, int j) const { return x / p[j]; }
 };
 struct DivFast {
-  const float* r;
-  bool bad;
-  __device__ inline float div(float x, const float* p, int j) {
-    unsigned int u;
-    __builtin_memcpy(&u, &x, sizeof(u));
-    bad |= ((u & 0x7fffffffu) - 0x1f800000u >= 0x40000000u) & (u != 0u);
-    const float q = x * r[j];
-    const float rem = fmaf(-q, p[j], x);
-    return fmaf(rem, r[j], q);
-  }
+  const double* r;
+  unsigned int tiny;
+  __device__ inline float div(float x, const float*, int j) { return div_recip(x, r[j], tiny); }
 };
 
 // aeif_cond_beta_multisynapse, src/aeif_cond_beta_multisynapse_kernel.h:165-226
@@ -89,13 +108,13 @@ struct DivFast {
 // ---------------------------------------------------------------------------
 // Right-hand side of a population: with uniform divisor parameters (UNI)
 // through DivFast, evaluated again with IEEE divisions when a lane of the
-// wave had a dividend outside DivFast's exact range.
+// wave has a subnormal quotient.
 template <class M, bool UNI>
-__device__ inline void rhs(const float* y, float* dy, const float* p, const float* r) {
+__device__ inline void rhs(const float* y, float* dy, const float* p, const double* r) {
   if constexpr (UNI) {
-    DivFast dv{r, false};
+    DivFast dv{r, ~0u};
     M::deriv(y, dy, p, dv);
-    if (__builtin_expect(__any(dv.bad), 0)) {
+    if (__builtin_expect(__any(tiny_noted(dv.tiny)), 0)) {
       DivIEEE di;
       M::deriv(y, dy, p, di);
     }
@@ -103,6 +122,13 @@ __device__ inline void rhs(const float* y, float* dy, const float* p, const floa
     DivIEEE di;
     M::deriv(y, dy, p, di);
   }
+}
+
+// err / eps through the double reciprocal (div_recip; a subnormal quotient
+// decides nothing: the error ratio is only compared and raised to a power
+// when above err_min)
+__device__ inline float div_eps(float err) {
+  return (float)((double)err * (1.0 / (double)ck::eps));
 }
 
 __device__ inline bool lagged_spike(int raw) { return ((unsigned int)raw >> 31) != 0; }
@@ -113,52 +139,53 @@ __device__ inline bool lagged_spike(int raw) { return ((unsigned int)raw >> 31) 
 // max_j |h sum_i e_i k_i[j]| / ys[j] (before the division by eps).  Each
 // stage's sum_i a_i k_i is accumulated with fma and added to y with one more
 // (y + h*(...)), the contracted pattern this build fixes for kernel and oracle.
-template <class M, class F>
-__device__ inline float rk5_try(const float* y, const float* k1, const float* ys, float h,
-                                float* yn, F&& deriv) {
+// C: where the tableau's coefficients are read from (CkConst, CkRegs).
+template <class M, class C, class F>
+__device__ inline float rk5_try(const C& c, const float* y, const float* k1, const float* ys,
+                                float h, float* yn, F&& deriv) {
   float k2[M::NV], k3[M::NV], k4[M::NV], k5[M::NV], k6[M::NV];
-  const float h21 = h * ck::a21;
+  const float h21 = h * c.a21;
 #pragma unroll
   for (int j = 0; j < M::NV; ++j) yn[j] = fmaf(h21, k1[j], y[j]);
   deriv(yn, k2);
 #pragma unroll
-  for (int j = 0; j < M::NV; ++j) yn[j] = fmaf(h, fmaf(ck::a32, k2[j], ck::a31 * k1[j]), y[j]);
+  for (int j = 0; j < M::NV; ++j) yn[j] = fmaf(h, fmaf(c.a32, k2[j], c.a31 * k1[j]), y[j]);
   deriv(yn, k3);
 #pragma unroll
   for (int j = 0; j < M::NV; ++j) {
-    float t = fmaf(ck::a42, k2[j], ck::a41 * k1[j]);
-    t = fmaf(ck::a43, k3[j], t);
+    float t = fmaf(c.a42, k2[j], c.a41 * k1[j]);
+    t = fmaf(c.a43, k3[j], t);
     yn[j] = fmaf(h, t, y[j]);
   }
   deriv(yn, k4);
 #pragma unroll
   for (int j = 0; j < M::NV; ++j) {
-    float t = fmaf(ck::a52, k2[j], ck::a51 * k1[j]);
-    t = fmaf(ck::a53, k3[j], t);
-    t = fmaf(ck::a54, k4[j], t);
+    float t = fmaf(c.a52, k2[j], c.a51 * k1[j]);
+    t = fmaf(c.a53, k3[j], t);
+    t = fmaf(c.a54, k4[j], t);
     yn[j] = fmaf(h, t, y[j]);
   }
   deriv(yn, k5);
 #pragma unroll
   for (int j = 0; j < M::NV; ++j) {
-    float t = fmaf(ck::a62, k2[j], ck::a61 * k1[j]);
-    t = fmaf(ck::a63, k3[j], t);
-    t = fmaf(ck::a64, k4[j], t);
-    t = fmaf(ck::a65, k5[j], t);
+    float t = fmaf(c.a62, k2[j], c.a61 * k1[j]);
+    t = fmaf(c.a63, k3[j], t);
+    t = fmaf(c.a64, k4[j], t);
+    t = fmaf(c.a65, k5[j], t);
     yn[j] = fmaf(h, t, y[j]);
   }
   deriv(yn, k6);
   float err = 0.0f;
 #pragma unroll
   for (int j = 0; j < M::NV; ++j) {
-    float t = fmaf(ck::b3, k3[j], ck::b1 * k1[j]);
-    t = fmaf(ck::b4, k4[j], t);
-    t = fmaf(ck::b6, k6[j], t);
+    float t = fmaf(c.b3, k3[j], c.b1 * k1[j]);
+    t = fmaf(c.b4, k4[j], t);
+    t = fmaf(c.b6, k6[j], t);
     yn[j] = fmaf(h, t, y[j]);
-    float e = fmaf(ck::e3, k3[j], ck::e1 * k1[j]);
-    e = fmaf(ck::e4, k4[j], e);
-    e = fmaf(ck::e5, k5[j], e);
-    e = fmaf(ck::e6, k6[j], e);
+    float e = fmaf(c.e3, k3[j], c.e1 * k1[j]);
+    e = fmaf(c.e4, k4[j], e);
+    e = fmaf(c.e5, k5[j], e);
+    e = fmaf(c.e6, k6[j], e);
     const float v = (h * e) / ys[j];
     err = fmaxf(err, fabsf(v));
   }
@@ -202,7 +229,7 @@ __global__ void __launch_bounds__(256) rk5_kernel(RK5Args a) {
       for (;;) {
         if (h > h_max) h = h_max;
         if (h < h_min) h = h_min;
-        err = rk5_try<M>(y, k1, ys, h, yn, [&](const float* yy, float* dd) {
+        err = rk5_try<M>(CkConst(), y, k1, ys, h, yn, [&](const float* yy, float* dd) {
           rhs<M, false>(yy, dd, p, nullptr);
         });
         err /= ck::eps;
@@ -266,7 +293,11 @@ __global__ void __launch_bounds__(256) rk5_kernel(RK5Args a) {
 // (ballot + lane rank; no atomics).  Per neuron the arithmetic is exactly
 // that of rk5_kernel.  UNI: every parameter except refractory_step is
 // uniform over the population, so parameters come from the kernel-argument
-// table and divisions by them use reciprocals (DivRecip, bit-identical).
+// table and divisions by them use reciprocals (DivFast, bit-identical).
+//
+// The waves that take the neurons about to spike (the previous launch listed
+// them) run the chain form instead of this loop (rk5_chain.h): one neuron
+// over a group of lanes.
 //
 // Step values of one persistent RK5 launch, read where they are used from
 // the launch's own kernel arguments (so the compiler reloads them instead of
@@ -320,10 +351,22 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
     flag_out = a.hot_flag + (size_t)(parity ^ 1) * n;
     if (wave == 0 && lane == 0) a.hot_count[q_clr] = 0;
   }
-  // wave w takes hot entries [w*hp, w*hp + hp) (one per lane, so the long
-  // attempt chains start together in the first iteration, packed into few
-  // waves), then its equal share of all neurons
-  const int hl = a.hot_lanes < 1 ? 1 : (a.hot_lanes > kWave ? kWave : a.hot_lanes);
+  // wave w takes hot entries [w*hp, w*hp + hp) (so the long attempt chains
+  // start together in the first iteration, packed into few waves), then its
+  // equal share of all neurons.  In the chain form a wave holds at most
+  // 64 / G entries; it takes fewer while there are waves to spread them over
+  // (neurons of one wave wait for each other's branches).
+  constexpr bool kChainOk = MODE == 0 && chain_capable<M>();
+  constexpr int kG = chain_lanes(M::NPORT);
+  bool chain = false;
+  int hl = a.hot_lanes < 1 ? 1 : (a.hot_lanes > kWave ? kWave : a.hot_lanes);
+  if constexpr (kChainOk) {
+    const int spread = a.chain_waves < n_waves / 2 ? a.chain_waves : n_waves / 2;
+    if (a.hot_only && spread > 0 && n_hot > 0 && n_hot <= (long long)spread * (kWave / kG)) {
+      chain = true;
+      hl = (n_hot + spread - 1) / spread;
+    }
+  }
   const int hp = n_hot <= (long long)n_waves * hl
                      ? hl
                      : (int)((((long long)n_hot + n_waves - 1) / n_waves + kWave - 1) & ~(long long)(kWave - 1));
@@ -353,8 +396,8 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   int pend = 0;         // bit 0: neuron finished this iteration, bit 1: it is hot
   int pend_i = 0;
   const float h_min = a.h_min;
-  const float r_eps = recip_rn(ck::eps);
-  float y[M::NV], p[M::NPAR], r[M::NPAR], k1[M::NV], ys[M::NV];
+  float y[M::NV], p[M::NPAR], k1[M::NV], ys[M::NV];
+  double r[M::NPAR];
   double x = 0.0;
   double cx1 = 0.0;     // end of the step the lane's neuron is in (x1, or x1_prev if lagged)
   bool lagged = false;
@@ -370,13 +413,198 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   float h_sub = 0.0f;   // controller proposal at the start of the substep
   bool clip = false;    // accepted attempt was cut by the end of the step
   bool rej_sub = false; // the current substep had a rejected attempt
-  unsigned long long n_att = 0, n_rej = 0, n_sub = 0;
-  unsigned int n_split = 0;
+  unsigned int n_att = 0, n_rej = 0, n_sub = 0, n_split = 0;
 #pragma unroll
   for (int j = 0; j < M::NPAR; ++j) {
     p[j] = a.tab.val[j];
-    r[j] = UNI ? recip_rn(p[j]) : 0.0f;
+    r[j] = UNI && M::divisor(j) ? recip_uniform(p[j]) : 0.0;
   }
+  // a spike that found the wave's buffer full: into the list at once
+  auto add_now = [&](int src_bits) {
+    spike_list_add(a.sl, lst, src_bits, 1.0f);
+    if (a.fd.lag_d0_at_exit && lagged_spike(src_bits)) {
+      // its d_int = 0 synapses now (the next launch folds their slot)
+      const int src = (int)((unsigned int)src_bits & ~kSpikeLagBit);
+      n_dev += deliver_segment(a.fd.st, spike_base_slot((unsigned int)src_bits, t_idx, a.fd.st.n_slot),
+                               1.0f, a.fd.st.row_ptr[src], a.fd.st.row_ptr[src + 1], 0, 1, 1);
+    }
+  };
+  if constexpr (kChainOk) {
+    if (chain && n_hw > 0) {
+      // ---- chain form: one neuron per group of kG lanes (rk5_chain.h) ----
+      const int role = lane & (kG - 1), k = role - 1;
+      const bool mem = role == 0, port = role >= 1 && role <= M::NPORT;
+      const int ia = mem ? M::iV : port ? M::c_ya(k) : -1;
+      const int ib = mem ? M::iw : port ? M::c_yb(k) : -1;
+      const bool busy0 = lane / kG < n_hw;
+      bool busy = busy0;
+      float ya[2] = {0.0f, 0.0f}, k1a[2] = {0.0f, 0.0f}, ysa[2] = {1.0f, 1.0f};
+      ChainDiv d{1.0f, 1.0f, 1.0f, 1.0, 1.0, 1.0};
+      double acc = 0.0;      // the port's stashed input while the neuron is lagged
+      float in_wt = 1.0f;    // weight of the port's input
+      if (busy0) {
+        i = dense[hs + lane / kG];
+        if (ia >= 0) ya[0] = a.var[(size_t)ia * n + i];
+        if (ib >= 0) ya[1] = a.var[(size_t)ib * n + i];
+        p[M::i_ref] = a.param[(size_t)M::i_ref * n + i];
+        if constexpr (!UNI) {
+#pragma unroll
+          for (int j = 0; j < M::NPAR; ++j)
+            if (a.tab.is_per_neuron(j)) p[j] = a.param[(size_t)j * n + i];
+        }
+        const int ja = mem ? M::c_mv : port ? M::c_da(k) : -1;
+        const int jb = mem ? M::c_mw : port ? M::c_db(k) : -1;
+        if (ja >= 0) d.da = a.param[(size_t)ja * n + i];
+        if (jb >= 0) d.db = a.param[(size_t)jb * n + i];
+        if (port && M::in_w(0) >= 0) in_wt = a.param[(size_t)M::in_w(k) * n + i];
+        x = a.x[i];
+        h = a.h[i];
+        lagged = a.lag ? a.lag[i] != 0 : false;
+        if (port) {
+          const long long lo = (long long)k * n;
+          if (sv.prefold()) {
+            const FoldArgs& f = a.pf;
+            double* rp = f.ring + (size_t)sv.pctx().slot * f.n_ch + (size_t)(f.ch_base + lo + i);
+            acc = poisson_input(f, lo + i, *rp, sv.pctx().t1, sv.pctx().t_idx,
+                                f.pu_b < lo + n && f.pu_e > lo);
+            *rp = 0.0;
+            constexpr int in = M::in_y(0) == M::c_ya(0) ? 0 : 1;
+            if (!lagged && acc != 0.0) ya[in] = fold_add(ya[in], acc, in_wt);
+          } else if (lagged) {
+            acc = a.pend[lo + i];
+          }
+        }
+        if (mem && a.sb.max_rec > 0) rec_k = a.sb.n_rec[i];
+        ref_in = p[M::i_ref];
+        if constexpr (M::c_mx >= 0) d.dx = p[M::c_mx < 0 ? 0 : M::c_mx];
+        cx1 = lagged ? x1_prev : x1;
+        need_k1 = true;
+        // the loads complete here, not in the loop
+        asm volatile("" ::"v"(ya[0]), "v"(ya[1]), "v"(ref_in), "v"(d.da), "v"(d.db), "v"(in_wt),
+                     "v"(x), "v"(h), "v"(acc), "v"(rec_k));
+      }
+      d.ra = recip_double(d.da);
+      d.rb = recip_double(d.db);
+      d.rx = recip_double(d.dx);
+      // (uniform populations: the launch checked the divisors)
+      const bool ieee = !UNI && __any(!(__builtin_isnormal(d.da) && __builtin_isnormal(d.db) &&
+                                        __builtin_isnormal(d.dx)));
+      CkRegs ckr;
+      ckr.hold();
+#pragma unroll
+      for (int j = 0; j < M::NPAR; ++j) asm volatile("" : "+v"(p[j]));
+      while (__any(busy)) {
+        if (busy) {
+          if (need_k1) {
+            unsigned int tiny = ieee ? 0u : ~0u;
+            chain_rhs<M, true>(ya, k1a, p, d, mem, tiny);
+            if (__builtin_expect(__any(tiny_noted(tiny)), 0)) chain_rhs<M, false>(ya, k1a, p, d, mem, tiny);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) ysa[j] = fabsf(ya[j]) + fabsf(k1a[j] * h) + ck::scal_min;
+            need_k1 = false;
+          }
+          const float h_max = (float)(cx1 - x);
+          if (h > h_max) h = h_max;
+          if (h < h_min) h = h_min;
+          float yn[2];
+          unsigned int tiny = ieee ? 0u : ~0u;
+          float err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, h, yn, [&](const float* yy, float* dd) {
+            chain_rhs<M, true>(yy, dd, p, d, mem, tiny);
+          });
+          if (__builtin_expect(__any(tiny_noted(tiny)), 0))
+            err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, h, yn, [&](const float* yy, float* dd) {
+              chain_rhs<M, false>(yy, dd, p, d, mem, tiny);
+            });
+          err = chain_max<kG>(err);
+          err = div_eps(err);
+          n_att += mem;
+          if (++att_i > kMaxAttempts) {   // non-finite state: end the step
+            x = cx1;
+            err = 0.0f;
+          }
+          const bool ok = err <= 1.0f || (double)h <= (double)h_min * (1.0 + 1.0e-5);
+          const float pw = pow_step_dev(err, ok, !ok || err > ck::err_min);
+          if (!ok) {
+            n_rej += mem;
+            const float h_new = h * ck::safety * pw;
+            h = (float)fmax((double)h_new, 0.1 * (double)h);
+          } else {
+            n_sub += mem;
+            if (att_i <= kMaxAttempts) x += h;
+            h = (err > ck::err_min) ? h * ck::safety * pw : 5.0f * h;
+            ya[0] = yn[0];
+            ya[1] = yn[1];
+            need_k1 = true;
+            const bool end_step = (x >= cx1 - (double)h_min);
+            if (mem) {
+              if (ya[0] < -1.0e3 || ya[1] < -1.0e6 || ya[1] > 1.0e6) {
+                ya[0] = p[M::i_reset];
+                ya[1] = 0.0f;
+              } else if (p[M::i_ref] > 0.0f) {
+                ya[0] = p[M::i_reset];
+                if (end_step) p[M::i_ref] -= 1.0f;
+              } else if (ya[0] >= p[M::i_thr]) {
+                spike_book(a.sb, a.i0 + i, i, 1.0f, lagged ? t_idx - 1 : t_idx, cx1, &rec_k);
+                spk = true;
+                spk_src = lagged ? (int)((unsigned int)(a.i0 + i) | kSpikeLagBit) : a.i0 + i;
+                ya[0] = p[M::i_reset];
+                ya[1] += p[M::i_jump];
+                const float rr = (float)(int)roundf(p[M::i_tref] / a.dt);
+                p[M::i_ref] = rr < 0.0f ? 0.0f : rr;
+              }
+            }
+            if (end_step && lagged) {
+              constexpr int in = M::in_y(0) == M::c_ya(0) ? 0 : 1;
+              if (port && acc != 0.0) ya[in] = fold_add(ya[in], acc, in_wt);
+              if (mem) a.lag[i] = 0;
+              lagged = false;
+              cx1 = x1;
+              att_i = 0;
+            } else if (end_step || (sv.defer_cap() > 0 && !lagged && att_i >= sv.defer_cap())) {
+              if (ia >= 0) a.var[(size_t)ia * n + i] = ya[0];
+              if (ib >= 0) a.var[(size_t)ib * n + i] = ya[1];
+              if (mem) {
+                if (!end_step) {
+                  a.lag[i] = 1;
+                  ++n_split;
+                }
+                a.x[i] = x;
+                a.h[i] = h;
+                if (p[M::i_ref] != ref_in) a.param[(size_t)M::i_ref * n + i] = p[M::i_ref];
+                pend = 1 | ((!end_step || (p[M::i_ref] <= 0.0f && ya[0] >= M::hot_v(p, a.hot_margin))) ? 2 : 0);
+                pend_i = i;
+              }
+              busy = false;
+            }
+          }
+        }
+        // spikes and hot entries of this iteration into the wave's buffers
+        // (at most 64 / kG neurons, so at most that many hot entries)
+        const unsigned long long ms = __ballot(spk);
+        if (ms) {
+          if (spk) {
+            const int pos = scnt + __popcll(ms & ((1ull << lane) - 1ull));
+            if (pos < kSpkLds) {
+              my_spk[pos] = spk_src;
+            } else {
+              add_now(spk_src);
+            }
+            spk = false;
+          }
+          scnt += __popcll(ms);
+        }
+        const unsigned long long mh = __ballot(pend == 3);
+        if (pend) {
+          if (pend == 3) my_hot[hcnt + __popcll(mh & ((1ull << lane) - 1ull))] = pend_i;
+          flag_out[pend_i] = pend == 3 ? 1 : 0;
+          pend = 0;
+        }
+        hcnt += __popcll(mh);
+      }
+      next = end;   // a chain wave takes no share of the bulk
+    }
+  }
+  if (!kChainOk || !(chain && n_hw > 0))
   for (;;) {
     // ---- refill idle lanes from the wave's chunk ----
     const bool want = (i < 0) && next < end;
@@ -511,10 +739,10 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       }
       if (h < h_min) h = h_min;
       float yn[M::NV];
-      float err = rk5_try<M>(y, k1, ys, h, yn, [&](const float* yy, float* dd) {
+      float err = rk5_try<M>(CkConst(), y, k1, ys, h, yn, [&](const float* yy, float* dd) {
         rhs<M, UNI>(yy, dd, p, r);
       });
-      err = div_rn(err, ck::eps, r_eps);
+      err = div_eps(err);
       ++n_att;
       if (++att_i > kMaxAttempts) {   // non-finite state: end the step (never hit by finite runs)
         x = cx1;
@@ -619,14 +847,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         if (pos < kSpkLds) {
           my_spk[pos] = spk_src;
         } else {
-          spike_list_add(a.sl, lst, spk_src, 1.0f);
-          if (a.fd.lag_d0_at_exit && lagged_spike(spk_src)) {
-            // its d_int = 0 synapses now (the next launch folds their slot)
-            const int src = (int)((unsigned int)spk_src & ~kSpikeLagBit);
-            n_dev += deliver_segment(a.fd.st, spike_base_slot((unsigned int)spk_src, t_idx,
-                                                              a.fd.st.n_slot),
-                                     1.0f, a.fd.st.row_ptr[src], a.fd.st.row_ptr[src + 1], 0, 1, 1);
-          }
+          add_now(spk_src);
         }
         spk = false;
       }
@@ -733,13 +954,13 @@ __device__ inline void clear_next_spike_list(const SpikeList& sl, int lst) {
   sl.count[lst == kSpikeLists - 1 ? 0 : lst + 1] = 0;
 }
 
-// Register budget of a small model's kernel (at most 6 state variables): the
-// plain kernel is held to 128 VGPRs (4 waves per SIMD) and the
-// learned-proposal kernel to 168 (3 waves); the compiler would otherwise take
-// a few more and drop a wave per SIMD.
+// Register budget of a small model's kernel (at most 6 state variables): 168
+// VGPRs, 3 waves per SIMD.  The chain form keeps the tableau and the
+// parameters in vector registers; held to 128 VGPRs (4 waves) it spilled 51
+// of them, and the bulk of a launch runs as fast with 3 waves as with 4.
 template <class M, bool UNI, int MODE>
 __global__ void __launch_bounds__(kRK5Block)
-__attribute__((amdgpu_waves_per_eu(M::NV > 6 ? 1 : MODE == 2 ? 3 : MODE == 0 ? 4 : 1)))
+__attribute__((amdgpu_waves_per_eu(M::NV <= 6 && MODE != 1 ? 3 : 1)))
 rk5_persistent_kernel(RK5Args a) {
   __shared__ int s_hot[kRK5Block / kWave][kHotLds];
   __shared__ int s_spk[kRK5Block / kWave][kSpkLds];

@@ -18,6 +18,16 @@
 // parameter that weights it (-1: weight 1), src/*.cu Init
 // (port_input_arr_, port_weight_arr_); hot_v the potential from which a
 // neuron is scheduled first in the next step (spike upswing).
+//
+// Chain form (rk5_chain.h), one neuron over 1 + NPORT lanes: the membrane
+// lane holds (V, w), port lane k the port's variables a (conductance or
+// current) and b (its rise variable, c_yb = -1 if the model has none);
+// c_ya(k) / c_yb(k) their indices, c_da(k) / c_db(k) the divisor parameters
+// of a / da and b / db; db/dt = -(b / db), da/dt = b - a / da (or -(a / da)).
+// c_mem gives the membrane lane's two numerators for the effective potential
+// V from the ports' a (ga(k)), the dividends of parameters c_mv and c_mw (or,
+// where these are -1, dV/dt and dw/dt themselves); c_mx is the divisor of
+// its inner division divx (-1: none).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -37,17 +47,16 @@ enum AdexTail { aV_th, aDelta_T, ag_L, aE_L, aC_m, aa, ab, atau_w, aI_e, aV_peak
 // first summed input term (fused into the g_L product) and I_2 the rest
 // (has_i2 false: "- w" follows the product directly and is fused instead).
 // psc: the models that skip the exponential when Delta_T == 0.
-template <bool PSC, class D>
-__device__ inline void adex_vw(const float* p, float V_m, float w, float i1, float i2, bool has_i1,
-                               bool has_i2, float* dV, float* dw, D& dv) {
-  const float* q = p;
-  const float V = (q[aref] > 0) ? q[aV_reset] : fminf(V_m, q[aV_peak]);
+// adex_num: the two numerators (dividends of C_m and tau_w) for the effective
+// potential V; divx(x) is x / Delta_T.
+template <bool PSC, class DX>
+__device__ inline void adex_num(const float* q, float V, float w, float i1, float i2, bool has_i1,
+                                bool has_i2, DX&& divx, float* num_v, float* num_w) {
   float V_spike;
   if (PSC) {
-    V_spike = q[aDelta_T] == 0.0f ? 0.0f
-                                  : q[aDelta_T] * exp_fma(dv.div(V - q[aV_th], q, aDelta_T));
+    V_spike = q[aDelta_T] == 0.0f ? 0.0f : q[aDelta_T] * exp_fma(divx(V - q[aV_th]));
   } else {
-    V_spike = q[aDelta_T] * exp_fma(dv.div(V - q[aV_th], q, aDelta_T));
+    V_spike = q[aDelta_T] * exp_fma(divx(V - q[aV_th]));
   }
   float num;
   if (has_i1) {
@@ -57,8 +66,20 @@ __device__ inline void adex_vw(const float* p, float V_m, float w, float i1, flo
   } else {
     num = fmaf(-q[ag_L], V - q[aE_L] - V_spike, -w) + q[aI_e];
   }
-  *dV = (q[aref] > 0) ? 0.0f : dv.div(num, q, aC_m);
-  *dw = dv.div(fmaf(q[aa], V - q[aE_L], -w), q, atau_w);
+  *num_v = num;
+  *num_w = fmaf(q[aa], V - q[aE_L], -w);
+}
+
+template <bool PSC, class D>
+__device__ inline void adex_vw(const float* p, float V_m, float w, float i1, float i2, bool has_i1,
+                               bool has_i2, float* dV, float* dw, D& dv) {
+  const float* q = p;
+  const float V = (q[aref] > 0) ? q[aV_reset] : fminf(V_m, q[aV_peak]);
+  float nv, nw;
+  adex_num<PSC>(q, V, w, i1, i2, has_i1, has_i2, [&](float x) { return dv.div(x, q, aDelta_T); },
+                &nv, &nw);
+  *dV = (q[aref] > 0) ? 0.0f : dv.div(nv, q, aC_m);
+  *dw = dv.div(nw, q, atau_w);
 }
 
 // Membrane potential of the AdEx models as their Derivatives see it.
@@ -81,6 +102,21 @@ struct AeifCondBeta {
   // input of port k: variable g1_k, weight g0_k (src/aeif_cond_beta_multisynapse.cu:151-159)
   static constexpr int in_y(int k) { return 3 + 2 * k; }
   static constexpr int in_w(int k) { return 14 + 4 * k + 3; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = Delta_T, c_mv = C_m, c_mw = tau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return 2 + 2 * k; }
+  __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
+  __host__ __device__ static constexpr int c_da(int k) { return 14 + 4 * k + 2; }
+  __host__ __device__ static constexpr int c_db(int k) { return 14 + 4 * k + 1; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    const float V = adex_v(p, V_m);
+    float I_syn = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) I_syn = fmaf(ga(i), p[14 + 4 * i] - V, I_syn);
+    adex_num<false>(p, V, w, I_syn, 0.0f, true, false, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     float I_syn = 0.0f;
@@ -115,6 +151,21 @@ struct AeifCondAlpha {
   // input of port k: variable g1_k, weight g0_k
   static constexpr int in_y(int k) { return 3 + 2 * k; }
   static constexpr int in_w(int k) { return 14 + 3 * k + 2; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = Delta_T, c_mv = C_m, c_mw = tau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return 2 + 2 * k; }
+  __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
+  __host__ __device__ static constexpr int c_da(int k) { return 14 + 3 * k + 1; }
+  __host__ __device__ static constexpr int c_db(int k) { return 14 + 3 * k + 1; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    const float V = adex_v(p, V_m);
+    float I_syn = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) I_syn = fmaf(ga(i), p[14 + 3 * i] - V, I_syn);
+    adex_num<false>(p, V, w, I_syn, 0.0f, true, false, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     float I_syn = 0.0f;
@@ -149,6 +200,20 @@ struct AeifPscExp {
     return j == tau_ex || j == tau_in || j == Delta_T || j == C_m || j == tau_w;
   }
   __device__ static inline float hot_v(const float* p, float m) { return fmaf(m, p[Delta_T], p[V_th]); }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = Delta_T, c_mv = C_m, c_mw = tau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return k; }
+  __host__ __device__ static constexpr int c_yb(int) { return -1; }
+  __host__ __device__ static constexpr int c_da(int k) { return tau_ex + k; }
+  __host__ __device__ static constexpr int c_db(int k) { return tau_ex + k; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w_, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    const float* q = p + V_th;
+    float I = 0.0f;
+    I += ga(0) - ga(1);
+    adex_num<true>(q, adex_v(q, V_m), w_, I, 0.0f, true, false, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     float I_syn_tot = 0.0f;
@@ -193,6 +258,21 @@ struct AeifCond2 {
   }
   static constexpr int in_y(int k) { return g1_ex + k; }
   static constexpr int in_w(int k) { return g0_ex + k; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = LEAD + aDelta_T, c_mv = LEAD + aC_m, c_mw = LEAD + atau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return g_ex + k; }
+  __host__ __device__ static constexpr int c_yb(int k) { return g1_ex + k; }
+  __host__ __device__ static constexpr int c_da(int k) { return tau_d(k); }
+  __host__ __device__ static constexpr int c_db(int k) { return tau_r(k); }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m_, float w_, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    const float* q = p + LEAD;
+    const float V = adex_v(q, V_m_);
+    const float I_ex = fmaf(ga(0), p[E_rev_ex] - V, 0.0f);
+    const float I_in = fmaf(ga(1), p[E_rev_in] - V, 0.0f);
+    adex_num<false>(q, V, w_, I_ex, I_in, true, true, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     const float* q = p + LEAD;
@@ -234,6 +314,20 @@ struct AeifPscAlpha {
   }
   static constexpr int in_y(int k) { return I1_ex + k; }
   static constexpr int in_w(int k) { return I0_ex + k; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = LEAD + aDelta_T, c_mv = LEAD + aC_m, c_mw = LEAD + atau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return I_ex + k; }
+  __host__ __device__ static constexpr int c_yb(int k) { return I1_ex + k; }
+  __host__ __device__ static constexpr int c_da(int k) { return tau_ex + k; }
+  __host__ __device__ static constexpr int c_db(int k) { return tau_ex + k; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m_, float w_, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    const float* q = p + LEAD;
+    float I = 0.0f;
+    I += ga(0) - ga(1);
+    adex_num<true>(q, adex_v(q, V_m_), w_, I, 0.0f, true, false, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     const float* q = p + LEAD;
@@ -267,6 +361,20 @@ struct AeifPscAlphaMS {
   __device__ static inline float hot_v(const float* p, float m) { return fmaf(m, p[aDelta_T], p[aV_th]); }
   static constexpr int in_y(int k) { return 3 + 2 * k; }
   static constexpr int in_w(int k) { return kAdexTail + 2 * k + 1; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = aDelta_T, c_mv = aC_m, c_mw = atau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return 2 + 2 * k; }
+  __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
+  __host__ __device__ static constexpr int c_da(int k) { return kAdexTail + 2 * k; }
+  __host__ __device__ static constexpr int c_db(int k) { return kAdexTail + 2 * k; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    float I = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) I += ga(i);
+    adex_num<true>(p, adex_v(p, V_m), w, I, 0.0f, true, false, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     float I_syn_tot = 0.0f;
@@ -295,6 +403,20 @@ struct AeifPscExpMS {
   __device__ static inline float hot_v(const float* p, float m) { return fmaf(m, p[aDelta_T], p[aV_th]); }
   static constexpr int in_y(int k) { return 2 + k; }
   static constexpr int in_w(int) { return -1; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = aDelta_T, c_mv = aC_m, c_mw = atau_w;
+  __host__ __device__ static constexpr int c_ya(int k) { return 2 + k; }
+  __host__ __device__ static constexpr int c_yb(int) { return -1; }
+  __host__ __device__ static constexpr int c_da(int k) { return kAdexTail + k; }
+  __host__ __device__ static constexpr int c_db(int k) { return kAdexTail + k; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+                                      float* nv, float* nw) {
+    float I = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) I += ga(i);
+    adex_num<true>(p, adex_v(p, V_m), w, I, 0.0f, true, false, divx, nv, nw);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     float I_syn_tot = 0.0f;
@@ -317,6 +439,8 @@ struct AeifPscDelta {
   __device__ static inline float hot_v(const float* p, float m) { return fmaf(m, p[aDelta_T], p[aV_th]); }
   static constexpr int in_y(int) { return 0; }
   static constexpr int in_w(int) { return -1; }
+  // every port feeds V_m: there are no port variables to give lanes to
+  static constexpr bool kChain = false;
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     adex_vw<true>(p, y[0], y[1], 0.0f, 0.0f, false, false, &dy[0], &dy[1], dv);
@@ -335,6 +459,22 @@ struct IzhCondBeta {
                        i_tref = t_ref, i_ref = ref;
   static constexpr bool divisor(int j) { return j >= 9 && (j - 9) % 4 >= 1 && (j - 9) % 4 <= 2; }
   __device__ static inline float hot_v(const float*, float) { return -45.0f; }
+  static constexpr bool kChain = true;
+  static constexpr int c_mx = -1, c_mv = -1, c_mw = -1;
+  __host__ __device__ static constexpr int c_ya(int k) { return 2 + 2 * k; }
+  __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
+  __host__ __device__ static constexpr int c_da(int k) { return 9 + 4 * k + 2; }
+  __host__ __device__ static constexpr int c_db(int k) { return 9 + 4 * k + 1; }
+  template <class G, class DX>
+  __device__ static inline void c_mem(const float* p, float V_m, float u, G&& ga, DX&&, float* dV,
+                                      float* du) {
+    float I_syn = 0.0f;
+    const float V = (p[ref] > 0) ? p[c] : V_m;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) I_syn = fmaf(ga(i), p[9 + 4 * i] - V, I_syn);
+    *dV = (float)(0.04 * V * V + 5.0 * V + 140.0 - u + I_syn + p[I_e]);
+    *du = p[a] * fmaf(p[b], V, -u);
+  }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
     float I_syn = 0.0f;
