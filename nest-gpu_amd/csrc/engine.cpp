@@ -2572,6 +2572,15 @@ void Engine::build_tiled(const std::vector<unsigned int>& ch, const std::vector<
   }
   upload(d_tsched_, sched, stream_);
   sync_streams();
+  {
+    // spikes of a step whose expected events stay below the sparse limit
+    int emitters = 0;
+    for (int s = 0; s < n_nodes_; ++s)
+      emitters += has_out_[s] && groups_[node_group_[s]]->md->id != MODEL_POISSON_GEN;
+    long long limit = tiled_env_ > 0 ? 0 : kTileSparseEvents;   // NGPU_TILED=1: tiles in every step
+    if (const char* env = getenv("NGPU_TILE_SPARSE")) limit = std::max(0ll, atoll(env));
+    tile_sparse_spk_ = (int)std::min<long long>(limit * std::max(emitters, 1) / (long long)nc, 1 << 30);
+  }
   tile_ch_ = tc;
   tile_rows_ = rows;
   n_tiles_ = (int)nt;
@@ -2591,6 +2600,8 @@ void Engine::deliver_list(const StepCtx& sc, const SpikeList& sl, int skip_lagge
     ta.tile_ev = d_tev_.p; ta.plan = d_tplan_.p; ta.sched = d_tsched_.p;
     ta.blocks = tiled_blocks_;
     ta.split_min = tile_split_min_;
+    ta.st = syn_table();
+    ta.sparse_spk = tile_sparse_spk_;
     timed(KT_DELIVER, [&] { launch_deliver_tiled(ta, stream_); });
     return;
   }

@@ -385,6 +385,7 @@ class Engine {
   DBuf<uint2> d_tplan_;               // work items of the next step
   DBuf<int> d_tsched_;                // {items, next item, finished blocks, 0}
   int tiled_blocks_ = 0;              // persistent grid of the tiled delivery
+  int tile_sparse_spk_ = 0;           // spikes of a step up to which it uses global atomics (NGPU_TILE_SPARSE: events)
   int tile_split_min_ = kTileSplitMin;  // NGPU_TILE_SPLIT_MIN
   bool defer_ok_ = false;              // inside Simulate() and not its last step
   int rk5_max_blocks_ = 1024;
@@ -396,7 +397,7 @@ class Engine {
   int batch_variant_ = 0;              // register budget: 0 = 3 waves per SIMD, 1 = 4
   int batch_iaf_unroll_ = 2;           // iaf_psc_exp neurons per lane per pass
   float batch_rk5_weight_ = 4.0f;      // blocks per RK5 neuron and state variable, relative to iaf
-  bool batch_graph_on_ = true;         // replay the launch as a HIP graph node
+  bool batch_graph_on_ = false;        // replay the launch as a HIP graph node (plan_batch says why not)
   int batch_grid_ = 0;
   std::vector<int> batch_groups_;      // group index of each batch population
   BatchArgs batch_plan_{};             // kinds and block partition

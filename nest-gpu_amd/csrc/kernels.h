@@ -287,12 +287,17 @@ struct TiledDeliverArgs {
   int* sched;                  // {items, next item, finished blocks}
   int blocks;                  // persistent grid
   int split_min;               // no split below this many events per item
+  SynTable st;                 // the source-major table, for steps with few spikes:
+  int sparse_spk;              // a step with at most this many is delivered by global atomics
 };
 void launch_deliver_tiled(const TiledDeliverArgs& a, hipStream_t s);
 // a tile is split over up to kTileSplitMax items; by default no split below
 // kTileSplitMin events per item
 constexpr int kTileSplitMax = 16;
 constexpr int kTileSplitMin = 16384;
+// events of a step (spikes x mean out-degree) up to which the tiled kernel
+// delivers by global atomics instead (kSparseEvents in kernels.hip says why)
+constexpr int kTileSparseEvents = 300000;
 // LDS bytes of one tile block at most (tile_ch * rows * 8): two blocks of
 // 16 waves fill a CU's 160 KB; tile_ch a multiple of 8, at most
 // kTileChMax; delay slots below 256 (the record's delay byte)

@@ -322,6 +322,41 @@ __device__ inline void tiled_plan(const TiledDeliverArgs& a) {
   }
 }
 
+// A step with few spikes: its events are added into the ring by global
+// atomics straight from the source-major table (the sums are the same bits),
+// the launch's waves sharing each spike's segment.  The tiles' chain of
+// dependent round trips (item, sources, runs, records, ring) and the plan
+// cost 21-30 us however few events there are, this form ~5 us and 1 us per
+// ~23,000 events.  The plan of the last dense step stays for the next one
+// (any plan covers every tile and spike).
+__device__ inline void tiled_sparse_step(const TiledDeliverArgs& a, int n_spk, const int* srcs,
+                                         const float* hts) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int n_waves = gridDim.x * (blockDim.x / kWave);
+  // consecutive blocks (different XCDs and CUs) take different spikes
+  const int wave = wv * gridDim.x + blockIdx.x;
+  const int parts = n_spk > 0 ? max(1, n_waves / n_spk) : 1;
+  unsigned long long n_ev = 0;
+  for (int w = wave; w < n_spk * parts; w += n_waves) {
+    const int s = w % n_spk, q = w / n_spk;
+    const unsigned int raw = (unsigned int)srcs[s];
+    const int src = (int)(raw & ~kSpikeLagBit);
+    const int mode = (a.skip_lagged_d0 && (raw >> 31)) ? 2 : 0;
+    n_ev += deliver_segment(a.st, spike_base_slot(raw, a.ctx.t_idx, a.st.n_slot), hts[s],
+                            a.st.row_ptr[src], a.st.row_ptr[src + 1], q * kWave + lane,
+                            parts * kWave, mode);
+  }
+  n_ev = wave_sum(n_ev);
+  if (lane == 0 && a.ctr && n_ev)
+    atomicAdd(&a.ctr[(size_t)(wave % kCtrMinRows) * kCtrCols + 3], n_ev);
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    if (a.spikes && n_spk) *a.spikes += (unsigned long long)n_spk;
+    const int lst = a.ctx.lst;
+    a.sl.count[lst == kSpikeLists - 1 ? 0 : lst + 1] = 0;
+  }
+}
+
 // at most 64 VGPRs: two 16-wave blocks per CU
 __global__ void __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
 deliver_tiled_kernel(TiledDeliverArgs a) {
@@ -340,6 +375,10 @@ deliver_tiled_kernel(TiledDeliverArgs a) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int n_wv = blockDim.x / kWave;
+  if (n_spk <= a.sparse_spk) {
+    tiled_sparse_step(a, n_spk, srcs, hts);
+    return;
+  }
   const int n_items = a.sched[0];
   const size_t row = (size_t)a.ts.n_tiles;
   // tiles can outnumber the counter rows: the waves add their counts into

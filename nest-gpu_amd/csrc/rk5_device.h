@@ -356,7 +356,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   // equal share of all neurons.  In the chain form a wave holds at most
   // 64 / G entries; it takes fewer while there are waves to spread them over
   // (neurons of one wave wait for each other's branches).
-  constexpr bool kChainOk = MODE == 0 && chain_capable<M>();
+  constexpr bool kChainOk = MODE != 1 && chain_capable<M>();
   constexpr int kG = chain_lanes(M::NPORT);
   bool chain = false;
   int hl = a.hot_lanes < 1 ? 1 : (a.hot_lanes > kWave ? kWave : a.hot_lanes);
@@ -475,13 +475,14 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           }
         }
         if (mem && a.sb.max_rec > 0) rec_k = a.sb.n_rec[i];
+        if constexpr (MODE == 2) el = a.err_last[i];
         ref_in = p[M::i_ref];
         if constexpr (M::c_mx >= 0) d.dx = p[M::c_mx < 0 ? 0 : M::c_mx];
         cx1 = lagged ? x1_prev : x1;
         need_k1 = true;
         // the loads complete here, not in the loop
         asm volatile("" ::"v"(ya[0]), "v"(ya[1]), "v"(ref_in), "v"(d.da), "v"(d.db), "v"(in_wt),
-                     "v"(x), "v"(h), "v"(acc), "v"(rec_k));
+                     "v"(x), "v"(h), "v"(acc), "v"(rec_k), "v"(el));
       }
       d.ra = recip_double(d.da);
       d.rb = recip_double(d.db);
@@ -494,6 +495,27 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
 #pragma unroll
       for (int j = 0; j < M::NPAR; ++j) asm volatile("" : "+v"(p[j]));
       while (__any(busy)) {
+        if constexpr (MODE == 2) {
+          // learned proposal, as in the loop below; the membrane lanes hold
+          // the neurons' inputs (columns of the matrix product)
+          const bool start = busy && need_k1 && h < (float)(cx1 - x);
+          if (__any(start)) {
+            float yy[M::NV], raw[kPI];
+            yy[0] = ya[0];
+            yy[1] = ya[1];
+#pragma unroll
+            for (int q = 0; q < M::NPORT; ++q) {
+              yy[2 + 2 * q] = chain_from(ya[0], q + 1);
+              yy[3 + 2 * q] = chain_from(ya[1], q + 1);
+            }
+            pred_raw_inputs<M::NPORT>(yy, h, el, a.dt, raw);
+#pragma unroll
+            for (int q = 0; q < kPI; ++q) raw[q] = busy && mem ? raw[q] : 0.0f;
+            const float o = __shfl(pred_infer_wave(*s_pred_p, raw), lane & ~(kG - 1), kWave);
+            if (start && o > -60.0f && o < 60.0f)
+              h = fminf(h, fmaxf(a.dt * exp2f(o), 2.0f * h_min));
+          }
+        }
         if (busy) {
           if (need_k1) {
             unsigned int tiny = ieee ? 0u : ~0u;
@@ -530,6 +552,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
             h = (float)fmax((double)h_new, 0.1 * (double)h);
           } else {
             n_sub += mem;
+            if constexpr (MODE == 2) el = err;
             if (att_i <= kMaxAttempts) x += h;
             h = (err > ck::err_min) ? h * ck::safety * pw : 5.0f * h;
             ya[0] = yn[0];
@@ -570,6 +593,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
                 }
                 a.x[i] = x;
                 a.h[i] = h;
+                if constexpr (MODE == 2) a.err_last[i] = el;
                 if (p[M::i_ref] != ref_in) a.param[(size_t)M::i_ref * n + i] = p[M::i_ref];
                 pend = 1 | ((!end_step || (p[M::i_ref] <= 0.0f && ya[0] >= M::hot_v(p, a.hot_margin))) ? 2 : 0);
                 pend_i = i;
@@ -748,17 +772,12 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         x = cx1;
         err = 0.0f;
       }
-      // the step factor of either branch: with a predictor (whose kernel
-      // already holds more registers) evaluated once for the wave; the plain
-      // kernel keeps one power per branch (the merged form costs it a
-      // register spill in the refill)
-      float pw = 0.0f;
-      if constexpr (MODE != 0)
-        pw = pow_step(err, err <= 1.0f || (double)h <= (double)h_min * (1.0 + 1.0e-5));
-      if (!(err <= 1.0f || (double)h <= (double)h_min * (1.0 + 1.0e-5))) {
+      const bool ok = err <= 1.0f || (double)h <= (double)h_min * (1.0 + 1.0e-5);
+      const float pw = pow_step_dev(err, ok, !ok || err > ck::err_min);
+      if (!ok) {
         ++n_rej;   // rejected: shrink h, retry with the same k1 and scale
         if constexpr (MODE == 1) rej_sub = true;
-        const float h_new = h * ck::safety * (MODE == 0 ? pow_m025(err) : pw);
+        const float h_new = h * ck::safety * pw;
         h = (float)fmax((double)h_new, 0.1 * (double)h);
       } else {
         ++n_sub;   // accepted (src/rk5.h:135-159), then ExternalUpdate
@@ -782,7 +801,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         }
         if constexpr (MODE != 0) el = err;
         if (att_i <= kMaxAttempts) x += h;
-        h = (err > ck::err_min) ? h * ck::safety * (MODE == 0 ? pow_m02(err) : pw) : 5.0f * h;
+        h = (err > ck::err_min) ? h * ck::safety * pw : 5.0f * h;
 #pragma unroll
         for (int j = 0; j < M::NV; ++j) y[j] = yn[j];
         need_k1 = true;
@@ -960,7 +979,7 @@ __device__ inline void clear_next_spike_list(const SpikeList& sl, int lst) {
 // of them, and the bulk of a launch runs as fast with 3 waves as with 4.
 template <class M, bool UNI, int MODE>
 __global__ void __launch_bounds__(kRK5Block)
-__attribute__((amdgpu_waves_per_eu(M::NV <= 6 && MODE != 1 ? 3 : 1)))
+__attribute__((amdgpu_waves_per_eu(M::NV > 6 || MODE == 1 ? 1 : MODE == 2 ? 2 : 3)))
 rk5_persistent_kernel(RK5Args a) {
   __shared__ int s_hot[kRK5Block / kWave][kHotLds];
   __shared__ int s_spk[kRK5Block / kWave][kSpkLds];
