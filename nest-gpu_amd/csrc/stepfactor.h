@@ -151,8 +151,9 @@ NGPU_HD inline float div_rn(float a, float d, float r) {
 // subnormal, overflowing to +inf above ~88.72).  Error < 1 ulp over the
 // whole float range (0.93 ulp at most; 99.5% of results correctly rounded).
 NGPU_HD inline float exp_fma(float x) {
-  // branch-free: the polynomial runs on the clamped argument and the special
-  // cases are selected afterwards (NaN -> x, above 100 -> +inf, below -110 -> 0)
+  // branch-free: the polynomial runs on the clamped argument; at the clamps
+  // the scaling itself overflows (e^100 > 2^128) or underflows to 0 (e^-110 <
+  // 2^-150), and NaN is selected afterwards
   const float xc = fminf(fmaxf(x, -110.0f), 100.0f);
   const float k = rintf(xc * 1.44269504f);
   float r = fmaf(-k, 0.693145752f, xc);
@@ -165,9 +166,7 @@ NGPU_HD inline float exp_fma(float x) {
   p = fmaf(p, r, 0.5f);
   p = fmaf(p, r, 1.0f);
   p = fmaf(p, r, 1.0f);
-  float e = ldexpf(p, (int)k);
-  e = x > 100.0f ? (float)INFINITY : e;
-  e = x < -110.0f ? 0.0f : e;
+  const float e = ldexpf(p, (int)k);
   return x == x ? e : x;
 }
 
