@@ -139,7 +139,7 @@ __device__ inline double poisson_input(const FoldArgs& f, long long idx, double 
     asm volatile("" ::"v"(origin), "v"(start), "v"(stop), "v"(chunks), "v"(e_chunk));
     const double t_rel = t1 - origin - f.pu_delay;
     if (in_run & (t_rel >= start) & (t_rel <= stop)) {
-      const int cnt = poisson_draw(f.seed, f.pu_stream0 + (unsigned int)r, t_idx, chunks, e_chunk);
+      const int cnt = poisson_draw_wave(f.seed, f.pu_stream0 + (unsigned int)r, t_idx, chunks, e_chunk);
       if (cnt > 0) acc += (double)(f.pu_w * (float)cnt);
     }
   } else if (f.pe_off) {
@@ -148,7 +148,8 @@ __device__ inline double poisson_input(const FoldArgs& f, long long idx, double 
       const int g = f.pe_gen[k];
       const double t_rel = t1 - f.gen_origin[g] - f.pe_delay[k];
       if (t_rel >= f.gen_start[g] && t_rel <= f.gen_stop[g]) {
-        const int cnt = poisson_draw(f.seed, f.pe_stream[k], t_idx, f.gen_chunks[g], f.gen_exp[g]);
+        const int cnt =
+            poisson_draw_wave(f.seed, f.pe_stream[k], t_idx, f.gen_chunks[g], f.gen_exp[g]);
         if (cnt > 0) acc += (double)(f.pe_w[k] * (float)cnt);
       }
     }
@@ -259,6 +260,60 @@ __device__ inline unsigned long long deliver_segment(const SynTable& t, int base
 __device__ inline int spike_base_slot(unsigned int raw, long long t_idx, int n_slot) {
   int b = (int)((t_idx + 1) % n_slot) - (int)(raw >> 31);
   return b < 0 ? b + n_slot : b;
+}
+
+// The d_int = 0 synapses of the lagged spikes among the n entries of a wave's
+// spike buffer (at most 64; height 1), by the whole wave: the entries' segment
+// bounds in one round trip, then one record per lane of kD0Batch spikes
+// before any atomic is issued (the d_int = 0 group heads the segment and
+// mostly has fewer than 64 records), so a wave waits for memory twice.
+constexpr int kD0Batch = 4;
+__device__ inline unsigned long long deliver_lagged_d0(const SynTable& t, const int* spk, int n,
+                                                       long long t_idx, int lane) {
+  unsigned long long n_ev = 0;
+  const unsigned int raw = lane < n ? (unsigned int)spk[lane] : 0u;
+  unsigned long long left = __ballot(raw >> 31);
+  if (!left) return 0;
+  long long b = 0, e = 0;
+  if (raw >> 31) {
+    const int src = (int)(raw & ~kSpikeLagBit);
+    b = t.row_ptr[src];
+    e = t.row_ptr[src + 1];
+  }
+  const int base = spike_base_slot(kSpikeLagBit, t_idx, t.n_slot);
+  while (left) {
+    unsigned int ch[kD0Batch];
+    float w[kD0Batch];
+    int d[kD0Batch];
+    long long kk[kD0Batch], en[kD0Batch];
+#pragma unroll
+    for (int q = 0; q < kD0Batch; ++q) {
+      d[q] = -1;
+      kk[q] = en[q] = 0;
+      if (left) {
+        const int from = __builtin_ctzll(left);
+        left &= left - 1;
+        kk[q] = __shfl(b, from, kWave) + lane;
+        en[q] = __shfl(e, from, kWave);
+        if (kk[q] < en[q]) {
+          ch[q] = t.syn_ch[kk[q]];
+          w[q] = t.syn_w[kk[q]];
+          d[q] = t.syn_d[kk[q]];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kD0Batch; ++q) {
+      if (d[q] == 0) {
+        unsafeAtomicAdd(&t.ring[(size_t)base * t.n_ch + ch[q]], (double)w[q]);
+        ++n_ev;
+      }
+      if (__shfl(d[q], kWave - 1, kWave) == 0)   // a longer group: the rest of it
+        n_ev += deliver_segment(t, base, 1.0f, __shfl(kk[q], kWave - 1, kWave) + 1, en[q], lane,
+                                kWave, 1);
+    }
+  }
+  return n_ev;
 }
 
 }  // namespace ngpu

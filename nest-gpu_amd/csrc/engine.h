@@ -371,12 +371,20 @@ class Engine {
   bool fused_deliver_ = false;         // ... and the network qualifies (one emitting RK5 population)
   bool prev_list_pending_ = false;     // the previous step's list awaits delivery by the next RK5 launch
   // lagged spikes' d_int = 0 synapses (fused delivery): 0 a launch after the
-  // update launch, 1 by the emitting wave at its exit
-  int lag_d0_mode_ = 0;
+  // update launch (5-7 us), 1 by the emitting wave at its exit (two round
+  // trips at the end of the chains: 84 -> 78 us a step on the 1e6-neuron
+  // network, 37 -> 34 on 1,000 neurons)
+  int lag_d0_mode_ = 1;
   // dense (tiled) delivery
   int tiled_env_ = -1;                 // NGPU_TILED: -1 when dense, 0 never, 1 whenever the table fits
   bool tiled_on_ = false;              // the tiled copy of the synapse table exists
   bool tiled_use_ = false;             // deliver with it (a batch autotuner knob)
+  bool tiled_auto_ = false;            // ... chosen per Simulate call (choose_delivery)
+  double events_per_spike_ = 0.0;      // mean out-degree of the emitters
+  unsigned long long call_spikes_ = 0; // spikes delivered before the last Simulate call
+  long long call_steps_ = 0;           // steps since
+  static constexpr double kFusedEvents = 100000.0;
+  void choose_delivery();
   int tile_ch_ = 0, n_tiles_ = 0, tile_rows_ = 0;
   int choose_tile_ch(int rows) const;
   DBuf<uint2> d_toff_;                // (first, end) record of each (source, tile)

@@ -553,13 +553,13 @@ void launch_deliver_tiled(const TiledDeliverArgs& a, hipStream_t s) {
 // synapses of the list's lagged spikes (their slot, t_emit + 1, is this
 // step's, which the next launch folds as its lanes take their neurons); the
 // rest of each lagged spike, and every other spike, is delivered with the
-// list by the next launch.  A wave takes kD0Batch list entries: lanes
-// 0..kD0Batch-1 load them together with the list's count, then the segment
+// list by the next launch.  A wave takes kListBatch list entries: lanes
+// 0..kListBatch-1 load them together with the list's count, then the segment
 // bounds of the lagged ones, then every lane loads one record of each (the
 // d_int = 0 group heads the segment and has far fewer than 64 records) before
 // any atomic is issued, so a wave waits for memory three times in all.
 constexpr int kLagD0Blocks = 64;
-constexpr int kD0Batch = 8;
+constexpr int kListBatch = 8;
 
 __global__ void __launch_bounds__(256) deliver_lagged_d0_kernel(DeliverArgs a) {
   const int lst = a.ctx.lst;
@@ -571,11 +571,11 @@ __global__ void __launch_bounds__(256) deliver_lagged_d0_kernel(DeliverArgs a) {
   const int n_waves = gridDim.x * (blockDim.x / kWave);
   const SynTable& t = a.st;
   unsigned long long n_ev = 0;
-  for (int e0 = wave * kD0Batch; e0 < cap; e0 += n_waves * kD0Batch) {
+  for (int e0 = wave * kListBatch; e0 < cap; e0 += n_waves * kListBatch) {
     // entries are read below the list's capacity whatever its count (the
     // count arrives with them; entries at or beyond it are masked after)
     const int e = e0 + lane;
-    const bool inb = lane < kD0Batch && e < cap;
+    const bool inb = lane < kListBatch && e < cap;
     unsigned int raw = 0u;
     float hgt = 0.0f;
     if (inb) {
@@ -594,12 +594,12 @@ __global__ void __launch_bounds__(256) deliver_lagged_d0_kernel(DeliverArgs a) {
       se = t.row_ptr[src + 1];
     }
     if (!__any(lg)) continue;
-    unsigned int ch[kD0Batch];
-    float w[kD0Batch];
-    int d[kD0Batch];
-    long long kk[kD0Batch];
+    unsigned int ch[kListBatch];
+    float w[kListBatch];
+    int d[kListBatch];
+    long long kk[kListBatch];
 #pragma unroll
-    for (int q = 0; q < kD0Batch; ++q) {
+    for (int q = 0; q < kListBatch; ++q) {
       const long long b = __shfl(sb, q, kWave), en = __shfl(se, q, kWave);
       kk[q] = b + lane;
       d[q] = -1;
@@ -610,7 +610,7 @@ __global__ void __launch_bounds__(256) deliver_lagged_d0_kernel(DeliverArgs a) {
       }
     }
 #pragma unroll
-    for (int q = 0; q < kD0Batch; ++q) {
+    for (int q = 0; q < kListBatch; ++q) {
       const int base = spike_base_slot(__shfl(raw, q, kWave), a.ctx.t_idx, t.n_slot);
       const float h = __shfl(hgt, q, kWave);
       if (d[q] == 0) {

@@ -77,4 +77,38 @@ NGPU_HD inline int poisson_draw(uint64_t seed, uint32_t stream, long long t_idx,
   return n;
 }
 
+#ifdef __HIPCC__
+// poisson_draw for all lanes of a wave together (lanes of a partly masked wave
+// too), the same counts.  With one chunk the count is the number of prefix
+// products that stay above the threshold (they only fall), so the uniforms of
+// a Philox block are taken without a branch: four multiplications, four
+// comparisons.  Blocks are wave-uniform, so the first rounds' products of the
+// counter's uniform words are scalar, and a wave goes on to the next block
+// while any lane is above its threshold (a mean of 2, 20 kHz at 0.1 ms: two
+// blocks).  The per-lane loop it replaces ran 7-9 rounds with ever fewer
+// lanes on, ~20 instructions each, and two to three Philox calls.
+__device__ inline int poisson_draw_wave(uint64_t seed, uint32_t stream, long long t_idx, int chunks,
+                                        double exp_chunk) {
+  if (__any(chunks > 1)) return poisson_draw(seed, stream, t_idx, chunks, exp_chunk);
+  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+  const uint32_t t_lo = (uint32_t)(uint64_t)t_idx, t_hi = (uint32_t)((uint64_t)t_idx >> 32);
+  double p = chunks > 0 ? 1.0 : 0.0;
+  const double e = chunks > 0 ? exp_chunk : 1.0;
+  int n = 0;
+  for (uint32_t blk = 0; __any(p > e); ++blk) {
+    const U32x4 r = philox4x32_10(U32x4{blk, t_lo, t_hi, stream}, k0, k1);
+    // ((double)r + 0.5) 2^-32, exact
+    p *= fma((double)r.x, 0x1p-32, 0x1p-33);
+    n += p > e;
+    p *= fma((double)r.y, 0x1p-32, 0x1p-33);
+    n += p > e;
+    p *= fma((double)r.z, 0x1p-32, 0x1p-33);
+    n += p > e;
+    p *= fma((double)r.w, 0x1p-32, 0x1p-33);
+    n += p > e;
+  }
+  return n;
+}
+#endif
+
 }  // namespace ngpu

@@ -340,51 +340,66 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   unsigned char* flag_out = nullptr;
   const int* dense = nullptr;
   int n_hot = 0, q_out = 0;
+  constexpr bool kChainOk = MODE != 1 && chain_capable<M>();
+  constexpr int kG = chain_lanes(M::NPORT);
+  // chain form: wave w < spread takes the hot entries w, w + spread, ... (one
+  // per group of lanes), so a launch with few of them gives each a wave of
+  // its own (neurons of one wave wait for each other's branches), and the
+  // entry is read together with the list's length
+  const int spread = kChainOk && a.hot_only ? (a.chain_waves < n_waves / 2 ? a.chain_waves : n_waves / 2) : 0;
+  const int my_entry = (lane / kG) * spread + wave;
+  int my_node = -1;
   if (a.hot_flag) {
     const int q_in = (int)(t_idx % 3);
     q_out = q_in == 2 ? 0 : q_in + 1;
     const int q_clr = q_out == 2 ? 0 : q_out + 1;   // read by the previous launch
+    dense = a.hot_list + (size_t)q_in * n;
+    if (wave < spread && my_entry < n) my_node = dense[my_entry];
     n_hot = a.hot_count[q_in];
     if (n_hot > n) n_hot = n;
-    dense = a.hot_list + (size_t)q_in * n;
     flag_in = a.hot_flag + (size_t)parity * n;
     flag_out = a.hot_flag + (size_t)(parity ^ 1) * n;
     if (wave == 0 && lane == 0) a.hot_count[q_clr] = 0;
   }
-  // wave w takes hot entries [w*hp, w*hp + hp) (so the long attempt chains
-  // start together in the first iteration, packed into few waves), then its
-  // equal share of all neurons.  In the chain form a wave holds at most
-  // 64 / G entries; it takes fewer while there are waves to spread them over
-  // (neurons of one wave wait for each other's branches).
-  constexpr bool kChainOk = MODE != 1 && chain_capable<M>();
-  constexpr int kG = chain_lanes(M::NPORT);
-  bool chain = false;
-  int hl = a.hot_lanes < 1 ? 1 : (a.hot_lanes > kWave ? kWave : a.hot_lanes);
-  if constexpr (kChainOk) {
-    const int spread = a.chain_waves < n_waves / 2 ? a.chain_waves : n_waves / 2;
-    if (a.hot_only && spread > 0 && n_hot > 0 && n_hot <= (long long)spread * (kWave / kG)) {
-      chain = true;
-      hl = (n_hot + spread - 1) / spread;
-    }
+  // without the chain form wave w takes hot entries [w*hp, w*hp + hp) (one
+  // per lane, so the long attempt chains start together in the first
+  // iteration, packed into few waves), then its equal share of all neurons
+  const bool chain = kChainOk && n_hot > 0 && n_hot <= spread * (kWave / kG);
+  int hs = 0, n_hw = 0, w_hot = 0;
+  if (chain) {
+    w_hot = n_hot < spread ? n_hot : spread;
+    n_hw = wave < w_hot ? 1 : 0;   // (the groups' entries are counted by my_entry)
+  } else if (n_hot > 0) {
+    const int hl = a.hot_lanes < 1 ? 1 : (a.hot_lanes > kWave ? kWave : a.hot_lanes);
+    const unsigned int hp =
+        n_hot <= n_waves * hl
+            ? (unsigned int)hl
+            : (((unsigned int)n_hot + n_waves - 1) / n_waves + kWave - 1) & ~(unsigned int)(kWave - 1);
+    hs = wave * (int)hp;
+    n_hw = hs < n_hot ? (hs + (int)hp < n_hot ? (int)hp : n_hot - hs) : 0;
+    w_hot = (int)(((unsigned int)n_hot + hp - 1) / hp);
   }
-  const int hp = n_hot <= (long long)n_waves * hl
-                     ? hl
-                     : (int)((((long long)n_hot + n_waves - 1) / n_waves + kWave - 1) & ~(long long)(kWave - 1));
-  const long long hs = (long long)wave * hp;
-  const int n_hw = hs < n_hot ? (int)((hs + hp < n_hot ? hs + hp : n_hot) - hs) : 0;
   // while the hot entries fill less than half the grid, the waves holding
   // them take no share of the bulk (a wave's bulk refills would stall its
-  // long chains on memory); the other waves split all neurons
-  const int w_hot = (int)(((long long)n_hot + hp - 1) / hp);
+  // long chains on memory); the other waves split all neurons, in units of
+  // 64, so that no wave has more than one unit more than another (a unit is
+  // one iteration: 1e6 neurons over 2,829 waves, 6 iterations in each at
+  // equal shares rounded up, 5 in half of them this way)
   const bool hot_only = a.hot_only && w_hot > 0 && 2 * w_hot <= n_waves;
-  const int n_bulk_waves = hot_only ? n_waves - w_hot : n_waves;
-  const long long bwave = hot_only ? (long long)wave - w_hot : (long long)wave;
-  const long long bchunk =
-      (((long long)n + n_bulk_waves - 1) / n_bulk_waves + kWave - 1) & ~(long long)(kWave - 1);
-  const long long b0 = bwave * bchunk;
-  const int n_bw = (bwave >= 0 && b0 < n) ? (int)((b0 + bchunk < n ? b0 + bchunk : n) - b0) : 0;
-  long long next = 0;
-  const long long end = (long long)n_hw + n_bw;
+  const int bwave = hot_only ? wave - w_hot : wave;
+  int b0 = 0, n_bw = 0;
+  if (bwave >= 0) {
+    const unsigned int nbw = hot_only ? n_waves - w_hot : n_waves;
+    const unsigned int units = ((unsigned int)n + kWave - 1) / kWave;
+    const unsigned int per = units / nbw, rem = units - per * nbw;
+    const unsigned int u0 = (unsigned int)bwave * per + ((unsigned int)bwave < rem ? bwave : rem);
+    const unsigned int u1 = u0 + per + ((unsigned int)bwave < rem ? 1u : 0u);
+    b0 = (int)(u0 * kWave);
+    const int b1 = (int)(u1 * kWave) < n ? (int)(u1 * kWave) : n;
+    n_bw = b1 > b0 ? b1 - b0 : 0;
+  }
+  int next = 0;
+  const int end = n_hw + n_bw;
   // the waves holding the chains issue first; the others fill the free slots
   if (n_hw > 0) __builtin_amdgcn_s_setprio(3);
   // spikes of the wave, appended to the step's list with one atomic when the
@@ -429,21 +444,24 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
                                1.0f, a.fd.st.row_ptr[src], a.fd.st.row_ptr[src + 1], 0, 1, 1);
     }
   };
+  CkRegs ckr;
+  if constexpr (M::NV <= 6) ckr.hold();
   if constexpr (kChainOk) {
     if (chain && n_hw > 0) {
+      if constexpr (M::NV > 6) ckr.hold();
       // ---- chain form: one neuron per group of kG lanes (rk5_chain.h) ----
       const int role = lane & (kG - 1), k = role - 1;
       const bool mem = role == 0, port = role >= 1 && role <= M::NPORT;
       const int ia = mem ? M::iV : port ? M::c_ya(k) : -1;
       const int ib = mem ? M::iw : port ? M::c_yb(k) : -1;
-      const bool busy0 = lane / kG < n_hw;
+      const bool busy0 = my_entry < n_hot;
       bool busy = busy0;
       float ya[2] = {0.0f, 0.0f}, k1a[2] = {0.0f, 0.0f}, ysa[2] = {1.0f, 1.0f};
       ChainDiv d{1.0f, 1.0f, 1.0f, 1.0, 1.0, 1.0};
       double acc = 0.0;      // the port's stashed input while the neuron is lagged
       float in_wt = 1.0f;    // weight of the port's input
       if (busy0) {
-        i = dense[hs + lane / kG];
+        i = my_node;
         if (ia >= 0) ya[0] = a.var[(size_t)ia * n + i];
         if (ib >= 0) ya[1] = a.var[(size_t)ib * n + i];
         p[M::i_ref] = a.param[(size_t)M::i_ref * n + i];
@@ -490,8 +508,6 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       // (uniform populations: the launch checked the divisors)
       const bool ieee = !UNI && __any(!(__builtin_isnormal(d.da) && __builtin_isnormal(d.db) &&
                                         __builtin_isnormal(d.dx)));
-      CkRegs ckr;
-      ckr.hold();
 #pragma unroll
       for (int j = 0; j < M::NPAR; ++j) asm volatile("" : "+v"(p[j]));
       // controller constants: the largest float h that passes the test
@@ -650,6 +666,11 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       next = end;   // a chain wave takes no share of the bulk
     }
   }
+  if constexpr (M::NV <= 6 && UNI) {
+#pragma unroll
+    for (int j = 0; j < M::NPAR; ++j)
+      if (M::divisor(j)) asm volatile("" : "+v"(r[j]));
+  }
   if (!kChainOk || !(chain && n_hw > 0))
   for (;;) {
     // ---- refill idle lanes from the wave's chunk ----
@@ -657,7 +678,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
     const unsigned long long m = __ballot(want);
     if (m) {
       if (want) {
-        const long long v = next + __popcll(m & ((1ull << lane) - 1ull));
+        const int v = next + __popcll(m & ((1ull << lane) - 1ull));
         // (written without a short-circuit on the flag: that form was
         // compiled with the candidate register overwritten by the flag address)
         int cand = -1;
@@ -665,7 +686,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           if (v < n_hw) {
             cand = dense[hs + v];
           } else {
-            const int b = (int)(b0 + (v - n_hw));
+            const int b = b0 + (v - n_hw);
             const int f = flag_in ? (int)flag_in[b] : 0;
             cand = f ? -1 : b;
           }
@@ -785,7 +806,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       }
       if (h < h_min) h = h_min;
       float yn[M::NV];
-      float err = rk5_try<M>(CkConst(), y, k1, ys, h, yn, [&](const float* yy, float* dd) {
+      float err = rk5_try<M>(ckr, y, k1, ys, h, yn, [&](const float* yy, float* dd) {
         rhs<M, UNI>(yy, dd, p, r);
       });
       err = div_eps(err);
@@ -929,20 +950,10 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           atomicAdd(a.sl.overflow, 1);
         }
       }
-      if (a.fd.lag_d0_at_exit) {
-        // the d_int = 0 synapses of the wave's lagged spikes: their slot
-        // (t_idx) is folded by the next launch; the other synapses are
-        // delivered with the list by the next launch's idle waves
-        for (int e = 0; e < listed; ++e) {
-          const int raw = my_spk[e];
-          if (!lagged_spike(raw)) continue;
-          const int src = (int)((unsigned int)raw & ~kSpikeLagBit);
-          n_dev += deliver_segment(a.fd.st, spike_base_slot((unsigned int)raw, t_idx,
-                                                            a.fd.st.n_slot),
-                                   1.0f, a.fd.st.row_ptr[src], a.fd.st.row_ptr[src + 1], lane,
-                                   kWave, 1);
-        }
-      }
+      // the d_int = 0 synapses of the wave's lagged spikes: their slot
+      // (t_idx) is folded by the next launch; the other synapses are
+      // delivered with the list by the next launch's idle waves
+      if (a.fd.lag_d0_at_exit) n_dev += deliver_lagged_d0(a.fd.st, my_spk, listed, t_idx, lane);
     }
   }
   if (a.hot_flag) {
