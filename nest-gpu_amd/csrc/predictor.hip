@@ -5,10 +5,10 @@
 // pass evaluates what inference computes (bfloat16 inputs, W1, W2 and
 // layer-1 activations, FP32 accumulation); gradients pass straight through
 // the rounding to the FP32 master weights, which Adam updates.  Gradient
-// sums are deterministic: every block (one wavefront) stages the per-sample
-// vectors of 64 samples in LDS and lane L accumulates parameters L, L+64, ...
-// over the samples in a fixed order, blocks write rows of partial sums, and
-// the update kernel adds the rows in block order.
+// sums are deterministic: every block stages the per-sample vectors of 64
+// samples in LDS and thread L accumulates parameters L, L+512, ... over the
+// samples in a fixed order, blocks write rows of partial sums, and the
+// update kernel adds the rows in block order.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -53,18 +53,37 @@ void launch_pred_stats(const float* log, long long n, double* part, int grid, hi
   hipLaunchKernelGGL(pred_stats_kernel, dim3(grid), dim3(256), 0, s, log, n, part);
 }
 
-// ---- forward + backward, one wavefront per block ----------------------------
+// ---- forward + backward: 64 samples per block and round ----------------------
+// Eight waves share a round's samples (lane = sample): wave w computes hidden
+// units 4w .. 4w+3 of both layers and of the backward pass, the activations
+// going through LDS as rows [unit][sample] (written without bank conflicts,
+// read back in 16-byte pieces of 4 samples), then every thread accumulates
+// up to kOwn parameters.  Every sum keeps one fixed order (units, then
+// samples, then rounds), whatever the number of waves.
+// Bound: the dependent LDS reads and additions of a round, not the matrix
+// work (0.06 GFLOP a batch): on matrix cores the sums would change.  Batch
+// 8192 (128 blocks): 85 us with one wave per block, whose row-major LDS
+// writes hit one bank with all 64 lanes and which summed 22 parameters per
+// lane; 14 us this way.
+constexpr int kGradWaves = 8, kGradThreads = 64 * kGradWaves;
+constexpr int kGradUnits = kPH / kGradWaves;   // units per wave
+constexpr int kRow = 68;   // floats per [unit][sample] row: 16-byte pieces of consecutive rows in other banks
+
 struct GradLDS {
   float w1q[kPH * kPI], w2q[kPH * kPH], b1[kPH], b2[kPH], w3[kPH], mu[kPI], is[kPI];
   float b3;
-  float xq[64][kPI], h1q[64][kPH], dz1[64][kPH], dz2[64][kPH], h2[64][kPH], dout[64];
+  alignas(16) float xq[kPI][kRow];
+  alignas(16) float h1q[kPH][kRow], dz1[kPH][kRow], dz2[kPH][kRow], h2[kPH][kRow];
+  alignas(16) float dout[kRow], one[kRow];
 };
 
-__global__ void __launch_bounds__(64) pred_grad_kernel(PredGradArgs a) {
+__global__ void __launch_bounds__(kGradThreads) pred_grad_kernel(PredGradArgs a) {
   __shared__ GradLDS L;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int u0 = wv * kGradUnits;
   const float* P = a.params;
-  for (int k = lane; k < kPH * kPH; k += 64) {
+  for (int k = tid; k < kPH * kPH; k += kGradThreads) {
     L.w2q[k] = bf16_round(P[kPOffW2 + k]);
     if (k < kPH * kPI) L.w1q[k] = bf16_round(P[kPOffW1 + k]);
     if (k < kPH) {
@@ -76,14 +95,37 @@ __global__ void __launch_bounds__(64) pred_grad_kernel(PredGradArgs a) {
       L.mu[k] = P[kPOffMu + k];
       L.is[k] = P[kPOffIs + k];
     }
+    if (k < 64) L.one[k] = 1.0f;
   }
-  if (lane == 0) L.b3 = P[kPOffB3];
+  if (tid == 0) L.b3 = P[kPOffB3];
   __syncthreads();
 
-  constexpr int kOwn = (kPNTrain + 63) / 64;
+  // parameter p of the thread: gradient sum over samples of rowA[s] * rowB[s]
+  // (times one for the biases, exact)
+  constexpr int kOwn = (kPNTrain + kGradThreads - 1) / kGradThreads;
+  const float *ra[kOwn], *rb[kOwn];
   float acc[kOwn];
 #pragma unroll
-  for (int k = 0; k < kOwn; ++k) acc[k] = 0.0f;
+  for (int k = 0; k < kOwn; ++k) {
+    const int p = tid + kGradThreads * k;
+    acc[k] = 0.0f;
+    ra[k] = L.dout;
+    rb[k] = L.one;   // b3, and threads past the last parameter
+    if (p < kPH * kPI) {
+      ra[k] = L.dz1[p / kPI];
+      rb[k] = L.xq[p % kPI];
+    } else if (p < kPH * kPI + kPH) {
+      ra[k] = L.dz1[p - kPH * kPI];
+    } else if (p < kPH * kPI + kPH + kPH * kPH) {
+      const int q = p - kPH * kPI - kPH;
+      ra[k] = L.dz2[q / kPH];
+      rb[k] = L.h1q[q % kPH];
+    } else if (p < kPH * kPI + 2 * kPH + kPH * kPH) {
+      ra[k] = L.dz2[p - kPH * kPI - kPH - kPH * kPH];
+    } else if (p < kPNTrain - 1) {
+      rb[k] = L.h2[p - (kPH * kPI + 2 * kPH + kPH * kPH)];
+    }
+  }
   float loss = 0.0f;
   const float inv_b = 1.0f / (float)a.batch;
 
@@ -101,7 +143,8 @@ __global__ void __launch_bounds__(64) pred_grad_kernel(PredGradArgs a) {
       const unsigned long long r64 = ((unsigned long long)o.x << 32) | o.y;
       src = (long long)(r64 % (unsigned long long)a.n_log);
     }
-    float x[kPI], z1[kPH], h1[kPH], z2[kPH], dz2[kPH], dout = 0.0f;
+    // (every wave reads the samples: the same lines, without a barrier more)
+    float x[kPI], z1[kGradUnits], z2[kGradUnits], dout = 0.0f;
     float t = 0.0f;
     bool cens = false;
     if (src >= 0 && a.raw) {
@@ -120,23 +163,36 @@ __global__ void __launch_bounds__(64) pred_grad_kernel(PredGradArgs a) {
 #pragma unroll
       for (int i = 0; i < kPI; ++i) x[i] = 0.0f;
     }
+    if (wv == 0) {
 #pragma unroll
-    for (int o = 0; o < kPH; ++o) {
+      for (int i = 0; i < kPI; ++i) L.xq[i][lane] = x[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kGradUnits; ++u) {
+      const int o = u0 + u;
       float s = L.b1[o];
 #pragma unroll
       for (int i = 0; i < kPI; ++i) s += L.w1q[o * kPI + i] * x[i];
-      z1[o] = s;
-      h1[o] = bf16_round(s > 0.0f ? s : 0.0f);
+      z1[u] = s;
+      L.h1q[o][lane] = bf16_round(s > 0.0f ? s : 0.0f);
     }
-    float out = L.b3;
-#pragma unroll 4
-    for (int o = 0; o < kPH; ++o) {
-      float s = L.b2[o];
+    __syncthreads();
+    {
 #pragma unroll
-      for (int i = 0; i < kPH; ++i) s += L.w2q[o * kPH + i] * h1[i];
-      z2[o] = s;
-      out += L.w3[o] * (s > 0.0f ? s : 0.0f);
+      for (int u = 0; u < kGradUnits; ++u) z2[u] = L.b2[u0 + u];
+#pragma unroll 8
+      for (int i = 0; i < kPH; ++i) {
+        const float h = L.h1q[i][lane];
+#pragma unroll
+        for (int u = 0; u < kGradUnits; ++u) z2[u] += L.w2q[(u0 + u) * kPH + i] * h;
+      }
+#pragma unroll
+      for (int u = 0; u < kGradUnits; ++u) L.h2[u0 + u][lane] = z2[u] > 0.0f ? z2[u] : 0.0f;
     }
+    __syncthreads();
+    float out = L.b3;
+#pragma unroll 8
+    for (int o = 0; o < kPH; ++o) out += L.w3[o] * L.h2[o][lane];
     if (src >= 0) {
       const float e = out - t;
       if (!(cens && e > 0.0f)) {
@@ -145,71 +201,89 @@ __global__ void __launch_bounds__(64) pred_grad_kernel(PredGradArgs a) {
       }
     }
 #pragma unroll
-    for (int o = 0; o < kPH; ++o) {
-      dz2[o] = z2[o] > 0.0f ? dout * L.w3[o] : 0.0f;
-      L.dz2[lane][o] = dz2[o];
-      L.h2[lane][o] = z2[o] > 0.0f ? z2[o] : 0.0f;
-      L.h1q[lane][o] = h1[o];
-    }
-#pragma unroll 4
-    for (int i = 0; i < kPH; ++i) {
-      float s = 0.0f;
-#pragma unroll
-      for (int o = 0; o < kPH; ++o) s += dz2[o] * L.w2q[o * kPH + i];
-      L.dz1[lane][i] = z1[i] > 0.0f ? s : 0.0f;
-    }
-#pragma unroll
-    for (int i = 0; i < kPI; ++i) L.xq[lane][i] = x[i];
-    L.dout[lane] = dout;
+    for (int u = 0; u < kGradUnits; ++u)
+      L.dz2[u0 + u][lane] = z2[u] > 0.0f ? dout * L.w3[u0 + u] : 0.0f;
+    if (wv == 0) L.dout[lane] = dout;
     __syncthreads();
-    // lane accumulates parameters p = lane + 64 k over the 64 samples
+    {
+      float s[kGradUnits];
 #pragma unroll
-    for (int k = 0; k < kOwn; ++k) {
-      const int p = lane + 64 * k;
-      if (p >= kPNTrain) break;
-      float sum = 0.0f;
-      if (p < kPH * kPI) {
-        const int o = p / kPI, i = p % kPI;
-        for (int s = 0; s < 64; ++s) sum += L.dz1[s][o] * L.xq[s][i];
-      } else if (p < kPH * kPI + kPH) {
-        const int o = p - kPH * kPI;
-        for (int s = 0; s < 64; ++s) sum += L.dz1[s][o];
-      } else if (p < kPH * kPI + kPH + kPH * kPH) {
-        const int q = p - kPH * kPI - kPH, o = q / kPH, i = q % kPH;
-        for (int s = 0; s < 64; ++s) sum += L.dz2[s][o] * L.h1q[s][i];
-      } else if (p < kPH * kPI + 2 * kPH + kPH * kPH) {
-        const int o = p - kPH * kPI - kPH - kPH * kPH;
-        for (int s = 0; s < 64; ++s) sum += L.dz2[s][o];
-      } else if (p < kPNTrain - 1) {
-        const int i = p - (kPH * kPI + 2 * kPH + kPH * kPH);
-        for (int s = 0; s < 64; ++s) sum += L.dout[s] * L.h2[s][i];
-      } else {
-        for (int s = 0; s < 64; ++s) sum += L.dout[s];
+      for (int u = 0; u < kGradUnits; ++u) s[u] = 0.0f;
+#pragma unroll 8
+      for (int o = 0; o < kPH; ++o) {
+        const float g = L.dz2[o][lane];
+#pragma unroll
+        for (int u = 0; u < kGradUnits; ++u) s[u] += g * L.w2q[o * kPH + u0 + u];
       }
-      acc[k] += sum;
+#pragma unroll
+      for (int u = 0; u < kGradUnits; ++u) L.dz1[u0 + u][lane] = z1[u] > 0.0f ? s[u] : 0.0f;
     }
+    __syncthreads();
+    float sum[kOwn];
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) sum[k] = 0.0f;
+#pragma unroll 4
+    for (int s = 0; s < 64; s += 4) {
+#pragma unroll
+      for (int k = 0; k < kOwn; ++k) {
+        const float4 p = *reinterpret_cast<const float4*>(ra[k] + s);
+        const float4 q = *reinterpret_cast<const float4*>(rb[k] + s);
+        sum[k] += p.x * q.x;
+        sum[k] += p.y * q.y;
+        sum[k] += p.z * q.z;
+        sum[k] += p.w * q.w;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) acc[k] += sum[k];
     __syncthreads();
   }
 #pragma unroll
   for (int k = 0; k < kOwn; ++k) {
-    const int p = lane + 64 * k;
+    const int p = tid + kGradThreads * k;
     if (p < kPNTrain) a.gpart[(size_t)blockIdx.x * kPNTrain + p] = acc[k];
   }
+  if (wv == 0) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
-  if (lane == 0) a.lpart[blockIdx.x] = loss;
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+    if (lane == 0) a.lpart[blockIdx.x] = loss;
+  }
 }
 
 void launch_pred_grad(const PredGradArgs& a, int blocks, hipStream_t s) {
-  hipLaunchKernelGGL(pred_grad_kernel, dim3(blocks), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(pred_grad_kernel, dim3(blocks), dim3(kGradThreads), 0, s, a);
 }
 
 // ---- sum of the block rows, then Adam (or only the sum) ---------------------
-__global__ void __launch_bounds__(256) pred_update_kernel(PredUpdateArgs a) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+// A block takes 32 parameters: its threads read kUpdRows rows of them into
+// LDS at once, then one thread per parameter adds them in row order (the
+// loss sums as a further column of the last block).  Bound: the latency of
+// the row reads; one thread per parameter reading 128 rows one after the
+// other took 37 us, this 5 us.
+constexpr int kUpdCols = 32, kUpdRows = 128, kUpdThreads = 512;
+
+__global__ void __launch_bounds__(kUpdThreads) pred_update_kernel(PredUpdateArgs a) {
+  __shared__ float tile[kUpdRows][kUpdCols + 1];
+  const int col = threadIdx.x % kUpdCols, row0 = threadIdx.x / kUpdCols;
+  const int p = blockIdx.x * kUpdCols + col;   // p == kPNTrain: the loss
+  float g = 0.0f;
+  for (int b0 = 0; b0 < a.blocks; b0 += kUpdRows) {
+    const int nb = a.blocks - b0 < kUpdRows ? a.blocks - b0 : kUpdRows;
+    if (p <= kPNTrain) {
+#pragma unroll
+      for (int r = row0; r < kUpdRows; r += kUpdThreads / kUpdCols)
+        if (r < nb)
+          tile[r][col] = p < kPNTrain ? a.gpart[(size_t)(b0 + r) * kPNTrain + p] : a.lpart[b0 + r];
+    }
+    __syncthreads();
+    if (row0 == 0 && p <= kPNTrain) {
+#pragma unroll 16
+      for (int r = 0; r < nb; ++r) g += tile[r][col];
+    }
+    __syncthreads();
+  }
+  if (row0 != 0) return;
   if (p < kPNTrain) {
-    float g = 0.0f;
-    for (int b = 0; b < a.blocks; ++b) g += a.gpart[(size_t)b * kPNTrain + p];
     if (a.grad_out) a.grad_out[p] = g;
     if (a.lr > 0.0f) {
       const float m = a.beta1 * a.m[p] + (1.0f - a.beta1) * g;
@@ -219,16 +293,14 @@ __global__ void __launch_bounds__(256) pred_update_kernel(PredUpdateArgs a) {
       const float mh = m / a.bc1, vh = v / a.bc2;
       a.params[kPOffW1 + p] -= a.lr * mh / (sqrtf(vh) + a.eps);
     }
-  }
-  if (p == 0) {
-    float l = 0.0f;
-    for (int b = 0; b < a.blocks; ++b) l += a.lpart[b];
-    a.loss_out[0] = l / (float)a.batch;
+  } else if (p == kPNTrain) {
+    a.loss_out[0] = g / (float)a.batch;
   }
 }
 
 void launch_pred_update(const PredUpdateArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(pred_update_kernel, dim3((kPNTrain + 255) / 256), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(pred_update_kernel, dim3((kPNTrain + 1 + kUpdCols - 1) / kUpdCols),
+                     dim3(kUpdThreads), 0, s, a);
 }
 
 // ---- inference through the matrix-core path (the one the RK5 kernel uses) ---
