@@ -108,6 +108,27 @@ __device__ inline void spike_list_add(const SpikeList& sl, int lst, int src, flo
   }
 }
 
+// spike_list_add for the lanes of a wave that spike together (every active
+// lane calls it): one atomic for all of them.  1,600 spikes a step added one
+// by one to the list's counter cost the iaf_psc_exp update 6 us.
+__device__ inline void spike_list_add_wave(const SpikeList& sl, int lst, bool fire, int src,
+                                           float height) {
+  const unsigned long long m = __ballot(fire);
+  if (!m) return;
+  const int lane = threadIdx.x & (kWave - 1), lead = __builtin_ctzll(m);
+  int base = 0;
+  if (lane == lead) base = atomicAdd(&sl.count[lst], __popcll(m));
+  base = __builtin_amdgcn_readlane(base, lead);
+  if (!fire) return;
+  const int pos = base + __popcll(m & ((1ull << lane) - 1ull));
+  if (pos < sl.cap) {
+    sl.src[(size_t)lst * sl.cap + pos] = src;
+    sl.height[(size_t)lst * sl.cap + pos] = height;
+  } else {
+    atomicAdd(sl.overflow, 1);
+  }
+}
+
 __device__ inline void emit_spike(const SpikeList& sl, const SpikeBook& sb,
                                   int lst, int node, int rel, float height,
                                   long long t_idx, double t1, bool lag = false) {

@@ -1710,6 +1710,19 @@ int Engine::Calibrate() {
   if (bad_port) throw Error("Connection port index larger than the number of ports of the target");
   for (int s = 0; s < n_nodes_; ++s) has_out_[s] = row_ptr_[s + 1] > row_ptr_[s];
   n_slot_ = max_d_int_ + 2;
+  {
+    // mean out-degree of the spiking nodes
+    long long emitters = 0, syn = 0;
+    for (int s = 0; s < n_nodes_; ++s) {
+      if (!has_out_[s] || groups_[node_group_[s]]->md->id == MODEL_POISSON_GEN) continue;
+      ++emitters;
+      syn += row_ptr_[s + 1] - row_ptr_[s];
+    }
+    events_per_spike_ = emitters ? (double)syn / (double)emitters : 0.0;
+    deliver_parts_log2_ = 0;
+    while (deliver_parts_log2_ < 3 && events_per_spike_ >= 512.0 * (1 << deliver_parts_log2_))
+      ++deliver_parts_log2_;
+  }
   phase("channels");
   // device synapse table
   upload(d_row_ptr_, row_ptr_, stream_);
@@ -2044,6 +2057,7 @@ RK5Args Engine::rk5_args(Group& gr, const StepCtx& sc, const SpikeList& sl, cons
     a.fd.lag_d0_at_exit = lag_d0_mode_;
     a.fd.skip_lagged_d0 = 1;
     a.fd.st = syn_table();
+    a.fd.parts_log2 = deliver_parts_log2_;
     a.fd.spikes = d_stats_.p;
     a.clear_next_list = 1;
     if (prev_list_pending_) {
@@ -2215,12 +2229,13 @@ void Engine::batch_partition() {
     w[k] = (double)g->n * (g->md->rk5 ? batch_rk5_weight_ * (double)g->nv : 1.0);
     tot += w[k];
   }
-  // blocks beyond one lane per neuron are useless: cap each population
+  // one lane per neuron, and as many blocks again for the hot entries and
+  // the delivery (more are useless): cap each population
   std::vector<int> nb(np), cap(np);
   int used = 0;
   for (int k = 0; k < np; ++k) {
     const Group* g = groups_[batch_groups_[k]];
-    cap[k] = std::max(1, (g->n + kRK5Block - 1) / kRK5Block);
+    cap[k] = 2 * std::max(1, (g->n + kRK5Block - 1) / kRK5Block);
     nb[k] = std::min(cap[k], std::max(1, (int)std::floor((double)grid * w[k] / tot)));
     used += nb[k];
   }
@@ -2250,7 +2265,13 @@ void Engine::batch_partition() {
   b.blk0[0] = 0;
   for (int k = 0; k < np; ++k) {
     const Group* g = groups_[batch_groups_[k]];
-    b.kind[k] = batch_kind_of(g->md->id, g->n_port, batch_iaf_unroll_);
+    // iaf_psc_exp: two neurons per lane and pass (their loads in flight
+    // together) only where a wave has that many (7,717 neurons: 9.0 us a
+    // launch with one, 12.0 with two; 77,169 the same)
+    const int waves = nb[k] * (kRK5Block / kWave);
+    const int unroll = batch_iaf_unroll_ > 0 ? batch_iaf_unroll_
+                       : g->n > (long long)waves * kWave ? 2 : 1;
+    b.kind[k] = batch_kind_of(g->md->id, g->n_port, unroll);
     b.blk0[k + 1] = b.blk0[k] + nb[k];
   }
   batch_grid_ = b.blk0[np];
@@ -2312,6 +2333,7 @@ void Engine::batch_step(const StepCtx& sc, const SpikeList& sl) {
   b.fd.lag_d0_at_exit = fu ? lag_d0_mode_ : 0;
   b.fd.skip_lagged_d0 = 1;
   b.fd.st = syn_table();
+  b.fd.parts_log2 = deliver_parts_log2_;
   b.fd.spikes = d_stats_.p;
   if (fu && prev_list_pending_) {
     b.fd.enable = 1;
@@ -2369,7 +2391,7 @@ void Engine::batch_step(const StepCtx& sc, const SpikeList& sl) {
 void Engine::GetBatchConfig(int* cfg) {
   cfg[0] = batch_on_ && Predictor::get().mode() == 0 ? 1 : 0;
   cfg[1] = batch_variant_;
-  cfg[2] = batch_iaf_unroll_;
+  cfg[2] = batch_iaf_unroll_ > 0 ? batch_iaf_unroll_ : 2;
   cfg[3] = (int)std::lround(batch_rk5_weight_ * 100.0f);
   cfg[4] = batch_graph_on_ ? 1 : 0;
   cfg[5] = batch_on_ ? batch_grid_ : 0;
@@ -2575,13 +2597,9 @@ void Engine::build_tiled(const std::vector<unsigned int>& ch, const std::vector<
   sync_streams();
   {
     // spikes of a step whose expected events stay below the sparse limit
-    int emitters = 0;
-    for (int s = 0; s < n_nodes_; ++s)
-      emitters += has_out_[s] && groups_[node_group_[s]]->md->id != MODEL_POISSON_GEN;
     long long limit = tiled_env_ > 0 ? 0 : kTileSparseEvents;   // NGPU_TILED=1: tiles in every step
     if (const char* env = getenv("NGPU_TILE_SPARSE")) limit = std::max(0ll, atoll(env));
-    tile_sparse_spk_ = (int)std::min<long long>(limit * std::max(emitters, 1) / (long long)nc, 1 << 30);
-    events_per_spike_ = (double)nc / std::max(emitters, 1);
+    tile_sparse_spk_ = (int)std::min(limit / std::max(events_per_spike_, 1.0), (double)(1 << 30));
   }
   tile_ch_ = tc;
   tile_rows_ = rows;

@@ -380,7 +380,8 @@ class Engine {
   bool tiled_on_ = false;              // the tiled copy of the synapse table exists
   bool tiled_use_ = false;             // deliver with it (a batch autotuner knob)
   bool tiled_auto_ = false;            // ... chosen per Simulate call (choose_delivery)
-  double events_per_spike_ = 0.0;      // mean out-degree of the emitters
+  double events_per_spike_ = 0.0;      // mean out-degree of the spiking nodes
+  int deliver_parts_log2_ = 0;         // waves that may share a spike's segment (fused delivery)
   unsigned long long call_spikes_ = 0; // spikes delivered before the last Simulate call
   long long call_steps_ = 0;           // steps since
   static constexpr double kFusedEvents = 100000.0;
@@ -403,7 +404,7 @@ class Engine {
   bool batch_active_ = false;          // ... and this Simulate call uses it (predictor off)
   bool batch_fold_pending_ = false;    // the previous step's fold is left to the next batch launch
   int batch_variant_ = 0;              // register budget: 0 = 3 waves per SIMD, 1 = 4
-  int batch_iaf_unroll_ = 2;           // iaf_psc_exp neurons per lane per pass
+  int batch_iaf_unroll_ = 0;           // iaf_psc_exp neurons per lane per pass (0: by size, batch_partition)
   float batch_rk5_weight_ = 4.0f;      // blocks per RK5 neuron and state variable, relative to iaf
   bool batch_graph_on_ = false;        // replay the launch as a HIP graph node (plan_batch says why not)
   int batch_grid_ = 0;

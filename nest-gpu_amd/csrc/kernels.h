@@ -141,6 +141,7 @@ struct FusedDeliver {
   int skip_lagged_d0;    // the previous list's lagged spikes had their d_int = 0 synapses delivered
   int prev_lst;          // list index of the previous step
   long long prev_t_idx;  // its time index
+  int parts_log2;        // waves that may share a spike (log2): a segment of mean length has 256 records per part
   SynTable st;
   unsigned long long* spikes;  // delivered spikes (one add per launch) or null
 };
@@ -296,8 +297,10 @@ void launch_deliver_tiled(const TiledDeliverArgs& a, hipStream_t s);
 constexpr int kTileSplitMax = 16;
 constexpr int kTileSplitMin = 16384;
 // events of a step (spikes x mean out-degree) up to which the tiled kernel
-// delivers by global atomics instead (kSparseEvents in kernels.hip says why)
-constexpr int kTileSparseEvents = 300000;
+// delivers by global atomics instead: those took 6 us + 1 us per 22,500
+// events (178,000: 14 us, 1.24e6: 61), the tiles 24 us + 1 us per 60,000
+// (141,000: 25 us, 1.24e6: 44)
+constexpr int kTileSparseEvents = 600000;
 // LDS bytes of one tile block at most (tile_ch * rows * 8): two blocks of
 // 16 waves fill a CU's 160 KB; tile_ch a multiple of 8, at most
 // kTileChMax; delay slots below 256 (the record's delay byte)

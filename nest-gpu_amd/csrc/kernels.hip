@@ -122,8 +122,10 @@ __global__ void __launch_bounds__(256) iaf_kernel(IafArgs a) {
   }
   iex *= P(P11ex);
   iin *= P(P11in);
-  if (v >= P(Theta)) {
-    emit_spike(a.sl, a.sb, a.ctx.lst, a.i0 + i, i, 1.0f, a.ctx.t_idx, a.ctx.t1);
+  const bool fire = v >= P(Theta);
+  spike_list_add_wave(a.sl, a.ctx.lst, fire, a.i0 + i, 1.0f);
+  if (fire) {
+    spike_book(a.sb, a.i0 + i, i, 1.0f, a.ctx.t_idx, a.ctx.t1);
     v = P(V_reset);
     ref = (float)(int)roundf(P(t_ref) / a.dt);
   }

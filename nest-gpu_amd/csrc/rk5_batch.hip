@@ -104,8 +104,10 @@ __device__ inline void iaf_batch_body(const IafArgs& a, const FoldArgs& f, const
       }
       iex[u] *= P(P11ex, i);
       iin[u] *= P(P11in, i);
-      if (v[u] >= P(Theta, i)) {
-        emit_spike(a.sl, a.sb, b.ctx.lst, a.i0 + i, i, 1.0f, b.ctx.t_idx, b.ctx.t1);
+      const bool fire = v[u] >= P(Theta, i);
+      spike_list_add_wave(a.sl, b.ctx.lst, fire, a.i0 + i, 1.0f);
+      if (fire) {
+        spike_book(a.sb, a.i0 + i, i, 1.0f, b.ctx.t_idx, b.ctx.t1);
         v[u] = P(V_reset, i);
         ref[u] = (float)(int)roundf(P(t_ref, i) / a.dt);
       }

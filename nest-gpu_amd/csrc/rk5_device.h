@@ -976,10 +976,13 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   add_wave_counters(a.ctr, ctr_row, lane, n_att, n_rej, n_sub);
 }
 
-// Fused delivery: the previous step's spike list, one spike per wave at a
-// time, taken from the last wave of the launch down so that the first waves
-// (the hot ones, which end last) take none while there are fewer spikes than
-// waves.  Returns the synapses delivered by the lane.
+// Fused delivery: the previous step's spike list, taken from the last wave of
+// the launch down so that the first waves (the hot ones, which end last) take
+// none while there are fewer spikes than waves.  Few spikes with long segments
+// are shared by up to 2^parts_log2 waves each (the last half of the launch's
+// waves), so a segment takes one round of record loads instead of several one
+// after the other.  Returns the synapses delivered by the lane.
+
 __device__ inline unsigned long long deliver_prev_list(const FusedDeliver& fd, const SpikeList& sl,
                                                        int wave, int n_waves, int lane) {
   unsigned long long n_dev = 0;
@@ -988,12 +991,16 @@ __device__ inline unsigned long long deliver_prev_list(const FusedDeliver& fd, c
   if (n_prev > sl.cap) n_prev = sl.cap;
   const int* srcs = sl.src + (size_t)pl * sl.cap;
   const float* hts = sl.height + (size_t)pl * sl.cap;
-  for (int sp = n_waves - 1 - wave; sp < n_prev; sp += n_waves) {
+  int lg = 0;   // log2 of the parts
+  while (lg < fd.parts_log2 && ((long long)n_prev << (lg + 2)) <= n_waves) ++lg;
+  for (int it = n_waves - 1 - wave; it < n_prev << lg; it += n_waves) {
+    const int sp = it >> lg, part = it & ((1 << lg) - 1);
     const unsigned int raw = (unsigned int)srcs[sp];
     const int src = (int)(raw & ~kSpikeLagBit);
     const int mode = (fd.skip_lagged_d0 && (raw >> 31)) ? 2 : 0;
     n_dev += deliver_segment(fd.st, spike_base_slot(raw, fd.prev_t_idx, fd.st.n_slot), hts[sp],
-                             fd.st.row_ptr[src], fd.st.row_ptr[src + 1], lane, kWave, mode);
+                             fd.st.row_ptr[src], fd.st.row_ptr[src + 1], part * kWave + lane,
+                             kWave << lg, mode);
   }
   if (wave == 0 && lane == 0 && fd.spikes && n_prev) *fd.spikes += (unsigned long long)n_prev;
   return n_dev;
