@@ -66,6 +66,20 @@ __device__ inline float pow_step_fast(float x, bool five) {
   const double c = d * fma(d, five ? 0.12 : 0.15625, five ? 0.2 : 0.25);
   return (float)fma(y, c, y);
 }
+// The same of x = div_eps(e) with the start taken from e itself, so that the
+// logarithm does not wait for the division, and both powers' starts from one
+// logarithm (compared with pow_m02 / pow_m025 for every e).
+__device__ inline float pow_step_chain(float e, float x, bool five) {
+  const float l = __builtin_amdgcn_logf(e) + 19.931569f;   // log2(1 / 1e-6)
+  const float a = __builtin_amdgcn_exp2f(l * -0.2f), b = __builtin_amdgcn_exp2f(l * -0.25f);
+  const double y = (double)(five ? a : b), X = (double)x;
+  const double y2 = y * y;
+  const double y4 = y2 * y2;
+  const double yn = five ? y4 * y : y4;
+  const double d = fma(-X, yn, 1.0);
+  const double c = d * fma(d, five ? 0.12 : 0.15625, five ? 0.2 : 0.25);
+  return (float)fma(y, c, y);
+}
 __device__ inline float pow_step_dev(float x, bool five, bool need) {
   float r = pow_step_fast(x, five);
   if (__builtin_expect(__any(need && !(x >= kPowLo && x <= kPowHi)), 0)) {
@@ -189,6 +203,20 @@ __device__ inline unsigned long long wave_sum(unsigned long long v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
   return v;
+}
+
+// Sum over the wave's 64 lanes (all on) by DPP: row shifts, then the row
+// broadcasts; the total, below 2^32, in a scalar register.  ~100 cycles; the
+// 64-bit shuffles of wave_sum go through LDS, ~900.
+__device__ inline unsigned int wave_sum32(unsigned int v) {
+  int x = (int)v;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr 1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr 2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr 4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2, 3
+  return (unsigned int)__builtin_amdgcn_readlane(x, 63);
 }
 
 // Adds a wave's counters into its own slot of the per-wave counter array

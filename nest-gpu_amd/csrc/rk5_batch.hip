@@ -145,6 +145,7 @@ rk5_batch_kernel(BatchArgs b) {
   const int gwave = (int)blockIdx.x * kWpb + wib;
   const int g_waves = (int)gridDim.x * kWpb;
   if (b.clear_next_list && blockIdx.x == 0 && threadIdx.x == 0) clear_next_spike_list(b.sl, b.ctx.lst);
+  const int n_prev = b.fd.enable ? b.sl.count[b.fd.prev_lst] : 0;
   unsigned long long n_dev = 0;
   int* my_hot = s_hot[threadIdx.x / kWave];
   int* my_spk = s_spk[threadIdx.x / kWave];
@@ -158,10 +159,10 @@ rk5_batch_kernel(BatchArgs b) {
     case BK_IAF4: iaf_batch_body<4>(c_batch_iaf[p], c_batch_fold[p], b, wave, n_waves, lane); break;
     default: break;
   }
-  if (b.fd.enable) n_dev += deliver_prev_list(b.fd, b.sl, gwave, g_waves, lane);
+  if (b.fd.enable) n_dev += deliver_prev_list(b.fd, b.sl, n_prev, gwave, g_waves, lane);
   if (b.ctr) {
-    n_dev = wave_sum(n_dev);
-    if (lane == 0 && n_dev) b.ctr[(size_t)gwave * kCtrCols + 3] += n_dev;
+    const unsigned int ev = wave_sum32((unsigned int)n_dev);
+    if (lane == 0 && ev) atomicAdd(b.ctr + (size_t)gwave * kCtrCols + 3, (unsigned long long)ev);
   }
 }
 

@@ -519,6 +519,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         if ((double)h_crit > hc) h_crit = __uint_as_float(__float_as_uint(h_crit) - 1u);
       }
       double x_end = cx1 - (double)h_min;
+      const int cap = sv.defer_cap();
       // The arithmetic runs unmasked in all 64 lanes, groups without a (busy)
       // neuron on harmless values, and only what follows from it is selected
       // by `busy`: a wave whose EXEC mask holds fewer than 16 lanes issues
@@ -548,12 +549,12 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
               h = fminf(h, fmaxf(a.dt * exp2f(o), 2.0f * h_min));
           }
         }
+        unsigned int tiny = ieee ? 0u : ~0u;
         if (__any(fresh)) {
           float kn[2];
-          unsigned int tiny = ieee ? 0u : ~0u;
-          chain_rhs<M, true>(ya, kn, p, d, mem, tiny);
-          if (__builtin_expect(__any(fresh && tiny_noted(tiny)), 0))
-            chain_rhs<M, false>(ya, kn, p, d, mem, tiny);
+          unsigned int tk = ~0u;
+          chain_rhs<M, true>(ya, kn, p, d, mem, tk);
+          tiny = fresh ? min(tiny, tk) : tiny;
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             k1a[j] = fresh ? kn[j] : k1a[j];
@@ -565,23 +566,43 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         if (hh > h_max) hh = h_max;
         if (hh < h_min) hh = h_min;
         float yn[2];
-        unsigned int tiny = ieee ? 0u : ~0u;
         float err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, hh, yn, [&](const float* yy, float* dd) {
           chain_rhs<M, true>(yy, dd, p, d, mem, tiny);
         });
-        if (__builtin_expect(__any(busy && tiny_noted(tiny)), 0))
-          err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, hh, yn, [&](const float* yy, float* dd) {
-            chain_rhs<M, false>(yy, dd, p, d, mem, tiny);
-          });
-        err = div_eps(chain_max<kG>(err));
+        const float err0 = chain_max<kG>(err);
+        err = div_eps(err0);
+        bool ok = (err <= 1.0f) | (hh <= h_crit);
+        float pw = pow_step_chain(err0, err, ok);
+        att_i += busy;
         bool over = false;
-        if (busy && ++att_i > kMaxAttempts) {   // non-finite state: end the step
-          x = cx1;
-          err = 0.0f;
-          over = true;
+        // rare cases behind one branch: a subnormal quotient (all divisions
+        // again by IEEE), the attempt bound of a non-finite state, an error
+        // ratio outside the range of the fast step factor
+        const bool need = !ok | (err > ck::err_min);
+        const bool rare = busy & (tiny_noted(tiny) | (att_i > kMaxAttempts) |
+                                  (need & !((err >= kPowLo) & (err <= kPowHi))));
+        if (__builtin_expect(__any(rare), 0)) {
+          if (__any(busy & tiny_noted(tiny))) {
+            float kn[2];
+            chain_rhs<M, false>(ya, kn, p, d, mem, tiny);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              k1a[j] = fresh ? kn[j] : k1a[j];
+              ysa[j] = fresh ? fabsf(ya[j]) + fabsf(kn[j] * h) + ck::scal_min : ysa[j];
+            }
+            err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, hh, yn, [&](const float* yy, float* dd) {
+              chain_rhs<M, false>(yy, dd, p, d, mem, tiny);
+            });
+            err = div_eps(chain_max<kG>(err));
+          }
+          if (busy & (att_i > kMaxAttempts)) {   // non-finite state: end the step
+            x = cx1;
+            err = 0.0f;
+            over = true;
+          }
+          ok = (err <= 1.0f) | (hh <= h_crit);
+          pw = pow_step_dev(err, ok, busy & (!ok | (err > ck::err_min)));
         }
-        const bool ok = err <= 1.0f || hh <= h_crit;
-        const float pw = pow_step_dev(err, ok, busy && (!ok || err > ck::err_min));
         const bool done = busy && ok;   // accepted (src/rk5.h:135-159)
         n_att += busy && mem;
         n_rej += busy && mem && !ok;
@@ -596,10 +617,14 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         ya[1] = done ? yn[1] : ya[1];
         need_k1 = busy ? ok : need_k1;
         if constexpr (MODE == 2) el = done ? err : el;
-        if (!__any(done)) continue;
-        // ExternalUpdate
+        // events behind one branch: ExternalUpdate acts on the membrane, the
+        // step ends or is split
         const bool end_step = x >= x_end;
-        const bool m = done && mem;
+        const bool m = done & mem;
+        const bool ext = m & ((ya[0] < -1.0e3f) | (ya[0] >= p[M::i_thr]) |
+                              (fabsf(ya[1]) > 1.0e6f) | (p[M::i_ref] > 0.0f));
+        const bool split = (cap > 0) & !lagged & (att_i >= cap);
+        if (!__any(ext | (done & (end_step | split)))) continue;
         const bool off = m && (ya[0] < -1.0e3 || ya[1] < -1.0e6 || ya[1] > 1.0e6);
         const bool refr = m && !off && p[M::i_ref] > 0.0f;
         const bool fire = m && !off && !refr && ya[0] >= p[M::i_thr];
@@ -624,8 +649,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           scnt += __popcll(ms);
         }
         const bool resume = done && end_step && lagged;   // the previous step is complete
-        const bool leave = done && !resume &&
-                           (end_step || (sv.defer_cap() > 0 && !lagged && att_i >= sv.defer_cap()));
+        const bool leave = done && !resume && (end_step || split);
         if (__any(resume)) {
           constexpr int in = M::in_y(0) == M::c_ya(0) ? 0 : 1;
           if (resume) {
@@ -934,47 +958,49 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
     }
   }
   {
-    // the wave's spikes into the step's list (order within a list does not
-    // matter: delivery sums exactly)
-    const int listed = scnt < kSpkLds ? scnt : kSpkLds;
-    if (listed > 0) {
-      int base = 0;
-      if (lane == 0) base = atomicAdd(a.sl.count + lst, listed);
-      base = __shfl(base, 0, kWave);
-      for (int e = lane; e < listed; e += kWave) {
-        const int pos = base + e;
+    // the wave's spikes into the step's list and its hot entries into the
+    // next step's (one atomic each; the order within a list does not matter:
+    // delivery sums exactly, scheduling changes no arithmetic).  Both atomics
+    // and the lagged spikes' segment bounds are in flight together.
+    const int n_spk = scnt < kSpkLds ? scnt : kSpkLds;
+    const int n_list = hcnt < kHotLds ? hcnt : kHotLds;
+    int spk_base = 0, hot_base = 0;
+    if (lane == 0) {
+      if (n_spk > 0) spk_base = atomicAdd(a.sl.count + lst, n_spk);
+      if (n_list > 0) hot_base = atomicAdd(a.hot_count + q_out, n_list);
+    }
+    // the d_int = 0 synapses of the wave's lagged spikes: their slot (t_idx)
+    // is folded by the next launch; the other synapses are delivered with the
+    // list by the next launch's idle waves
+    if (a.fd.lag_d0_at_exit && n_spk > 0)
+      n_dev += deliver_lagged_d0(a.fd.st, my_spk, n_spk, t_idx, lane);
+    if (n_spk > 0) {
+      const int pos = __builtin_amdgcn_readfirstlane(spk_base) + lane;   // kSpkLds entries: one per lane
+      if (lane < n_spk) {
         if (pos < a.sl.cap) {
-          a.sl.src[(size_t)lst * a.sl.cap + pos] = my_spk[e];
+          a.sl.src[(size_t)lst * a.sl.cap + pos] = my_spk[lane];
           a.sl.height[(size_t)lst * a.sl.cap + pos] = 1.0f;
         } else {
           atomicAdd(a.sl.overflow, 1);
         }
       }
-      // the d_int = 0 synapses of the wave's lagged spikes: their slot
-      // (t_idx) is folded by the next launch; the other synapses are
-      // delivered with the list by the next launch's idle waves
-      if (a.fd.lag_d0_at_exit) n_dev += deliver_lagged_d0(a.fd.st, my_spk, listed, t_idx, lane);
+    }
+    if (n_list > 0) {
+      int* out = a.hot_list + (size_t)q_out * n + __builtin_amdgcn_readfirstlane(hot_base);
+      for (int e = lane; e < n_list; e += kWave) out[e] = my_hot[e];
+    }
+    if (a.ctr) {
+      // (no value is read back, so the wave does not wait)
+      const unsigned int c[5] = {wave_sum32(n_att), wave_sum32(n_rej), wave_sum32(n_sub),
+                                 (unsigned int)n_list, wave_sum32(n_split)};
+      unsigned long long* row = a.ctr + (size_t)ctr_row * kCtrCols;
+#pragma unroll
+      for (int k = 0; k < 5; ++k)
+        if (lane == 0 && c[k]) atomicAdd(row + (k < 3 ? k : k + 1), (unsigned long long)c[k]);
     }
   }
-  if (a.hot_flag) {
-    // append the wave's list to the next step's (one atomic per wave; the
-    // order of the entries only affects scheduling)
-    const int listed = hcnt < kHotLds ? hcnt : kHotLds;
-    if (listed > 0) {
-      int base = 0;
-      if (lane == 0) base = atomicAdd(a.hot_count + q_out, listed);
-      base = __shfl(base, 0, kWave);
-      int* out = a.hot_list + (size_t)q_out * n + base;
-      for (int e = lane; e < listed; e += kWave) out[e] = my_hot[e];
-      if (lane == 0 && a.ctr) a.ctr[(size_t)ctr_row * kCtrCols + 4] += (unsigned long long)listed;
-    }
-  }
-  if (a.lag && a.ctr) {
-    const unsigned long long ns = wave_sum(n_split);
-    if (lane == 0 && ns) a.ctr[(size_t)ctr_row * kCtrCols + 5] += ns;
-  }
-  add_wave_counters(a.ctr, ctr_row, lane, n_att, n_rej, n_sub);
 }
+static_assert(kSpkLds <= kWave, "one spike entry per lane when the wave's buffer is written out");
 
 // Fused delivery: the previous step's spike list, taken from the last wave of
 // the launch down so that the first waves (the hot ones, which end last) take
@@ -982,12 +1008,11 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
 // are shared by up to 2^parts_log2 waves each (the last half of the launch's
 // waves), so a segment takes one round of record loads instead of several one
 // after the other.  Returns the synapses delivered by the lane.
-
+// n_prev: the list's length, read when the launch began.
 __device__ inline unsigned long long deliver_prev_list(const FusedDeliver& fd, const SpikeList& sl,
-                                                       int wave, int n_waves, int lane) {
+                                                       int n_prev, int wave, int n_waves, int lane) {
   unsigned long long n_dev = 0;
   const int pl = fd.prev_lst;
-  int n_prev = sl.count[pl];
   if (n_prev > sl.cap) n_prev = sl.cap;
   const int* srcs = sl.src + (size_t)pl * sl.cap;
   const float* hts = sl.height + (size_t)pl * sl.cap;
@@ -1002,7 +1027,7 @@ __device__ inline unsigned long long deliver_prev_list(const FusedDeliver& fd, c
                              fd.st.row_ptr[src], fd.st.row_ptr[src + 1], part * kWave + lane,
                              kWave << lg, mode);
   }
-  if (wave == 0 && lane == 0 && fd.spikes && n_prev) *fd.spikes += (unsigned long long)n_prev;
+  if (wave == 0 && lane == 0 && fd.spikes && n_prev) atomicAdd(fd.spikes, (unsigned long long)n_prev);
   return n_dev;
 }
 
@@ -1034,13 +1059,14 @@ rk5_persistent_kernel(RK5Args a) {
   const int n_waves = gridDim.x * (blockDim.x / kWave);
   if (a.clear_next_list && blockIdx.x == 0 && threadIdx.x == 0) clear_next_spike_list(a.sl, a.ctx.lst);
   const StepFromArgs sv{a};
+  const int n_prev = a.fd.enable ? a.sl.count[a.fd.prev_lst] : 0;
   unsigned long long n_dev = 0;   // synapses delivered by this lane (fused delivery)
   rk5_persistent_body<M, UNI, MODE>(a, sv, wave, n_waves, wave, s_hot[threadIdx.x / kWave],
                                     s_spk[threadIdx.x / kWave], &s_pred, n_dev);
-  if (a.fd.enable) n_dev += deliver_prev_list(a.fd, a.sl, wave, n_waves, lane);
+  if (a.fd.enable) n_dev += deliver_prev_list(a.fd, a.sl, n_prev, wave, n_waves, lane);
   if (a.ctr) {
-    n_dev = wave_sum(n_dev);
-    if (lane == 0 && n_dev) a.ctr[(size_t)wave * kCtrCols + 3] += n_dev;
+    const unsigned int ev = wave_sum32((unsigned int)n_dev);
+    if (lane == 0 && ev) atomicAdd(a.ctr + (size_t)wave * kCtrCols + 3, (unsigned long long)ev);
   }
 }
 
