@@ -155,6 +155,7 @@ __device__ inline void emit_spike(const SpikeList& sl, const SpikeBook& sb,
 // by edge, src/poiss_gen.cu:55-86.  Poisson edges are sorted by channel, so
 // each lane sums its own edges (no atomics).  Contraction is off: the double
 // expressions round exactly as the reference's.
+template <bool kRekey = false>
 __device__ inline double poisson_input(const FoldArgs& f, long long idx, double acc, double t1,
                                        long long t_idx, bool run_here) {
 #pragma clang fp contract(off)
@@ -174,7 +175,7 @@ __device__ inline double poisson_input(const FoldArgs& f, long long idx, double 
     asm volatile("" ::"v"(origin), "v"(start), "v"(stop), "v"(chunks), "v"(e_chunk));
     const double t_rel = t1 - origin - f.pu_delay;
     if (in_run & (t_rel >= start) & (t_rel <= stop)) {
-      const int cnt = poisson_draw_wave(f.seed, f.pu_stream0 + (unsigned int)r, t_idx, chunks, e_chunk);
+      const int cnt = poisson_draw_wave<kRekey>(f.seed, f.pu_stream0 + (unsigned int)r, t_idx, chunks, e_chunk);
       if (cnt > 0) acc += (double)(f.pu_w * (float)cnt);
     }
   } else if (f.pe_off) {
@@ -184,7 +185,7 @@ __device__ inline double poisson_input(const FoldArgs& f, long long idx, double 
       const double t_rel = t1 - f.gen_origin[g] - f.pe_delay[k];
       if (t_rel >= f.gen_start[g] && t_rel <= f.gen_stop[g]) {
         const int cnt =
-            poisson_draw_wave(f.seed, f.pe_stream[k], t_idx, f.gen_chunks[g], f.gen_exp[g]);
+            poisson_draw_wave<kRekey>(f.seed, f.pe_stream[k], t_idx, f.gen_chunks[g], f.gen_exp[g]);
         if (cnt > 0) acc += (double)(f.pe_w[k] * (float)cnt);
       }
     }

@@ -87,15 +87,28 @@ NGPU_HD inline int poisson_draw(uint64_t seed, uint32_t stream, long long t_idx,
 // while any lane is above its threshold (a mean of 2, 20 kHz at 0.1 ms: two
 // blocks).  The per-lane loop it replaces ran 7-9 rounds with ever fewer
 // lanes on, ~20 instructions each, and two to three Philox calls.
+// kRekey: the key schedule is computed at each block, by the scalar unit.
+// For the RK5 kernels, where it would be hoisted out of the refill loop: its
+// 20 keys and first products then hold the scalar registers, and spilling
+// others costs more vector instructions than the schedule (1e6 AdEx neurons,
+// 67.3 -> 66.0 us a step together with the refill's single round trip).  The
+// iaf_psc_exp kernels have the registers (re-keyed, 77,169 neurons: 15.7 ->
+// 16.0 us).
+template <bool kRekey = false>
 __device__ inline int poisson_draw_wave(uint64_t seed, uint32_t stream, long long t_idx, int chunks,
                                         double exp_chunk) {
   if (__any(chunks > 1)) return poisson_draw(seed, stream, t_idx, chunks, exp_chunk);
-  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-  const uint32_t t_lo = (uint32_t)(uint64_t)t_idx, t_hi = (uint32_t)((uint64_t)t_idx >> 32);
+  auto word = [](uint64_t v) {
+    if constexpr (kRekey) return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    return (uint32_t)v;
+  };
+  uint32_t k0 = word(seed), k1 = word(seed >> 32);
+  uint32_t t_lo = word((uint64_t)t_idx), t_hi = word((uint64_t)t_idx >> 32);
   double p = chunks > 0 ? 1.0 : 0.0;
   const double e = chunks > 0 ? exp_chunk : 1.0;
   int n = 0;
   for (uint32_t blk = 0; __any(p > e); ++blk) {
+    if constexpr (kRekey) asm volatile("" : "+s"(k0), "+s"(k1), "+s"(t_lo), "+s"(t_hi));
     const U32x4 r = philox4x32_10(U32x4{blk, t_lo, t_hi, stream}, k0, k1);
     // ((double)r + 0.5) 2^-32, exact
     p *= fma((double)r.x, 0x1p-32, 0x1p-33);

@@ -147,8 +147,8 @@ rk5_batch_kernel(BatchArgs b) {
   if (b.clear_next_list && blockIdx.x == 0 && threadIdx.x == 0) clear_next_spike_list(b.sl, b.ctx.lst);
   const int n_prev = b.fd.enable ? b.sl.count[b.fd.prev_lst] : 0;
   unsigned long long n_dev = 0;
-  int* my_hot = s_hot[threadIdx.x / kWave];
-  int* my_spk = s_spk[threadIdx.x / kWave];
+  int* my_hot = s_hot[wib];
+  int* my_spk = s_spk[wib];
   switch (b.kind[p]) {
     case BK_COND_BETA2: batch_rk5<AeifCondBeta<2>>(b, p, wave, n_waves, gwave, my_hot, my_spk, n_dev); break;
     case BK_COND_ALPHA4: batch_rk5<AeifCondAlpha<4>>(b, p, wave, n_waves, gwave, my_hot, my_spk, n_dev); break;

@@ -13,13 +13,16 @@
 // the group by DPP.  Every variable goes through exactly the operations of
 // M::deriv, rk5_try and the persistent loop, so results are the same bits.
 //
-// Bound: the latency of one attempt's dependent instructions.  Measured
-// (MI355X, time of a 0.1 ms step, one lane per neuron -> chain form with the
-// reciprocal divisions and the step factor from hardware log2/exp2): 1e6
-// AdEx neurons with 100 synapses each, 13.9 Hz, 134 -> 89 us; 1,000 neurons
-// 65 -> 42 us; 1,000 with plastic synapses (no split steps, so the whole
-// chain in one launch) 109 -> 68 us; the six-population batch of 50,330
-// neurons 130 -> 70 us.
+// Bound: the latency of one attempt's dependent instructions, ~2,300 cycles
+// from one attempt to the next, 23 of them in a launch.  Measured (MI355X,
+// time of a 0.1 ms step, one lane per neuron -> this form): 1e6 AdEx neurons
+// with 100 synapses each, 13.9 Hz, 134 -> 66 us; 60,000 with 1,000 synapses
+// 120 -> 37.6 us; 1,000 neurons 65 -> 28.9 us; 2,000 with plastic synapses (no
+// split steps, so the whole chain in one launch) 105 -> 52.5 us; the
+// six-population batch of 50,330 neurons 127 -> 39.7 us.  Of these k1 taken
+// beside the error ratio, and the shorter right-hand side (ChainNote below,
+// the error ratio by reciprocal), gave 39.6 -> 37.6, 30.6 -> 28.9,
+// 55.7 -> 52.5 and 41.1 -> 39.7 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -77,29 +80,61 @@ struct ChainNV {
   static constexpr int NV = 2;   // variables per lane, as rk5_try counts them
 };
 
-// d(a, b)/dt of the lane's variables (FAST: divisions by reciprocal, smallest
-// subnormal quotient noted in tiny; else IEEE divisions)
+// What a lane's fast divisions and exponentials met that needs the IEEE form:
+// the smallest subnormal quotient (div_recip) and the largest exponent.
+struct ChainNote {
+  unsigned int tiny;
+  float big;
+  __device__ bool set() const { return tiny_noted(tiny) | !(big <= kExpNear); }
+};
+
+// d(a, b)/dt of the lane's variables.  FAST, on an attempt's serial path:
+// divisions by reciprocal; the potential's clamp as one median of three (a
+// NaN becomes -inf, which is noted); the exponential without its clamps, whose
+// argument is noted where these act beyond kExpNear (a subnormal argument
+// needs no note: exp is 1 either way); signs and the refractory zero as one
+// fma with the lane's sign and addend (1, -0: exact).  Else the IEEE form.
 template <class M, bool FAST>
 __device__ inline void chain_rhs(const float* y, float* dy, const float* p, const ChainDiv& d,
-                                 bool mem, unsigned int& tiny) {
+                                 bool mem, ChainNote& note) {
   constexpr bool kB = M::c_yb(0) >= 0;   // the ports have a rise variable
   auto quot = [&](float x, double r, float den) {
     if constexpr (FAST) {
-      return div_recip(x, r, tiny);
+      return div_recip(x, r, note.tiny);
     } else {
       return x / den;
     }
   };
+  const bool refr = p[M::i_ref] > 0.0f;
+  struct {
+    const ChainDiv& d;
+    ChainNote& note;
+    float lo, hi;
+    __device__ float v(const float* q, float V) const {
+      if constexpr (FAST) return __builtin_amdgcn_fmed3f(V, lo, hi);
+      return adex_v(q, V);
+    }
+    __device__ float expx(float x) const {
+      if constexpr (!FAST) return exp_fma(x / d.dx);
+      const float q = (float)((double)x * d.rx);
+      note.big = fmaxf(note.big, fabsf(q));
+      return exp_fma_near(q);
+    }
+  } fx{d, note, refr ? p[M::i_reset] : -__builtin_inff(), refr ? p[M::i_reset] : p[M::i_thr]};
   float nv, nw;
-  M::c_mem(p, y[0], y[1], [&](int k) { return chain_from(y[0], k + 1); },
-           [&](float x) { return quot(x, d.rx, d.dx); }, &nv, &nw);
-  const float qa = quot(M::c_mv >= 0 && mem ? nv : y[0], d.ra, d.da);
+  M::c_mem(p, y[0], y[1], [&](int k) { return chain_from(y[0], k + 1); }, fx, &nv, &nw);
   float qb = 0.0f;
   if constexpr (kB || M::c_mw >= 0) qb = quot(M::c_mw >= 0 && mem ? nw : y[1], d.rb, d.db);
-  const float ma = p[M::i_ref] > 0.0f ? 0.0f : (M::c_mv >= 0 ? qa : nv);
-  const float mb = M::c_mw >= 0 ? qb : nw;
-  dy[0] = mem ? ma : kB ? y[1] - qa : -qa;
-  dy[1] = mem ? mb : kB ? -qb : 0.0f;
+  dy[1] = mem ? (M::c_mw >= 0 ? qb : nw) : kB ? -qb : 0.0f;
+  if constexpr (FAST && M::c_mv >= 0) {
+    const bool move = mem && !refr;
+    const float ya = mem && refr ? 0.0f : y[0];
+    const float add = mem ? (refr ? 0.0f : -0.0f) : kB ? y[1] : -0.0f;
+    dy[0] = fmaf(mem ? 1.0f : -1.0f, quot(move ? nv : ya, d.ra, d.da), add);
+  } else {
+    const float qa = quot(M::c_mv >= 0 && mem ? nv : y[0], d.ra, d.da);
+    dy[0] = mem ? (refr ? 0.0f : (M::c_mv >= 0 ? qa : nv)) : kB ? y[1] - qa : -qa;
+  }
 }
 
 }  // namespace ngpu

@@ -96,11 +96,18 @@ struct CkRegs {
 // branch, normally not taken, per evaluation.
 struct DivIEEE {
   __device__ inline float div(float x, const float* p, int j) const { return x / p[j]; }
+  __device__ inline float exp_div(float x, const float* p, int j) const { return exp_fma(x / p[j]); }
 };
 struct DivFast {
   const double* r;
   unsigned int tiny;
+  bool far;   // an exponent outside exp_fma_near's range (a subnormal one: exp is 1 either way)
   __device__ inline float div(float x, const float*, int j) { return div_recip(x, r[j], tiny); }
+  __device__ inline float exp_div(float x, const float*, int j) {
+    const float q = (float)((double)x * r[j]);
+    far = !(fabsf(q) <= kExpNear);
+    return exp_fma_near(q);
+  }
 };
 
 // aeif_cond_beta_multisynapse, src/aeif_cond_beta_multisynapse_kernel.h:165-226
@@ -108,13 +115,13 @@ struct DivFast {
 // ---------------------------------------------------------------------------
 // Right-hand side of a population: with uniform divisor parameters (UNI)
 // through DivFast, evaluated again with IEEE divisions when a lane of the
-// wave has a subnormal quotient.
+// wave has a subnormal quotient or an exponent out of range.
 template <class M, bool UNI>
 __device__ inline void rhs(const float* y, float* dy, const float* p, const double* r) {
   if constexpr (UNI) {
-    DivFast dv{r, ~0u};
+    DivFast dv{r, ~0u, false};
     M::deriv(y, dy, p, dv);
-    if (__builtin_expect(__any(tiny_noted(dv.tiny)), 0)) {
+    if (__builtin_expect(__any(tiny_noted(dv.tiny) | dv.far), 0)) {
       DivIEEE di;
       M::deriv(y, dy, p, di);
     }
@@ -136,12 +143,13 @@ __device__ inline bool lagged_spike(int raw) { return ((unsigned int)raw >> 31) 
 // ---------------------------------------------------------------------------
 // One Cash-Karp attempt of step h from (y, k1), src/rk5.h:88-131: the five
 // further stages, the 5th-order solution yn and the error ratio
-// max_j |h sum_i e_i k_i[j]| / ys[j] (before the division by eps).  Each
+// max_j |h sum_i e_i k_i[j]| / ys[j] (before the division by eps; rel(v, j) is
+// v / ys[j]).  Each
 // stage's sum_i a_i k_i is accumulated with fma and added to y with one more
 // (y + h*(...)), the contracted pattern this build fixes for kernel and oracle.
 // C: where the tableau's coefficients are read from (CkConst, CkRegs).
-template <class M, class C, class F>
-__device__ inline float rk5_try(const C& c, const float* y, const float* k1, const float* ys,
+template <class M, class C, class Q, class F>
+__device__ inline float rk5_try(const C& c, const float* y, const float* k1, Q&& rel,
                                 float h, float* yn, F&& deriv) {
   float k2[M::NV], k3[M::NV], k4[M::NV], k5[M::NV], k6[M::NV];
   const float h21 = h * c.a21;
@@ -186,7 +194,7 @@ __device__ inline float rk5_try(const C& c, const float* y, const float* k1, con
     e = fmaf(c.e4, k4[j], e);
     e = fmaf(c.e5, k5[j], e);
     e = fmaf(c.e6, k6[j], e);
-    const float v = (h * e) / ys[j];
+    const float v = rel(h * e, j);
     err = fmaxf(err, fabsf(v));
   }
   return err;
@@ -229,7 +237,8 @@ __global__ void __launch_bounds__(256) rk5_kernel(RK5Args a) {
       for (;;) {
         if (h > h_max) h = h_max;
         if (h < h_min) h = h_min;
-        err = rk5_try<M>(CkConst(), y, k1, ys, h, yn, [&](const float* yy, float* dd) {
+        auto rel = [&](float v, int j) { return v / ys[j]; };
+        err = rk5_try<M>(CkConst(), y, k1, rel, h, yn, [&](const float* yy, float* dd) {
           rhs<M, false>(yy, dd, p, nullptr);
         });
         err /= ck::eps;
@@ -412,7 +421,6 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   int pend_i = 0;
   const float h_min = a.h_min;
   float y[M::NV], p[M::NPAR], k1[M::NV], ys[M::NV];
-  double r[M::NPAR];
   double x = 0.0;
   double cx1 = 0.0;     // end of the step the lane's neuron is in (x1, or x1_prev if lagged)
   bool lagged = false;
@@ -430,10 +438,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   bool rej_sub = false; // the current substep had a rejected attempt
   unsigned int n_att = 0, n_rej = 0, n_sub = 0, n_split = 0;
 #pragma unroll
-  for (int j = 0; j < M::NPAR; ++j) {
-    p[j] = a.tab.val[j];
-    r[j] = UNI && M::divisor(j) ? recip_uniform(p[j]) : 0.0;
-  }
+  for (int j = 0; j < M::NPAR; ++j) p[j] = a.tab.val[j];
   // a spike that found the wave's buffer full: into the list at once
   auto add_now = [&](int src_bits) {
     spike_list_add(a.sl, lst, src_bits, 1.0f);
@@ -458,7 +463,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       bool busy = busy0;
       float ya[2] = {0.0f, 0.0f}, k1a[2] = {0.0f, 0.0f}, ysa[2] = {1.0f, 1.0f};
       ChainDiv d{1.0f, 1.0f, 1.0f, 1.0, 1.0, 1.0};
-      double acc = 0.0;      // the port's stashed input while the neuron is lagged
+      double in_add = -0.0;  // the port's stashed input while the neuron is lagged (-0: none)
       float in_wt = 1.0f;    // weight of the port's input
       if (busy0) {
         i = my_node;
@@ -480,16 +485,22 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         lagged = a.lag ? a.lag[i] != 0 : false;
         if (port) {
           const long long lo = (long long)k * n;
+          double acc = 0.0;
           if (sv.prefold()) {
             const FoldArgs& f = a.pf;
             double* rp = f.ring + (size_t)sv.pctx().slot * f.n_ch + (size_t)(f.ch_base + lo + i);
-            acc = poisson_input(f, lo + i, *rp, sv.pctx().t1, sv.pctx().t_idx,
+            acc = poisson_input<true>(f, lo + i, *rp, sv.pctx().t1, sv.pctx().t_idx,
                                 f.pu_b < lo + n && f.pu_e > lo);
             *rp = 0.0;
-            constexpr int in = M::in_y(0) == M::c_ya(0) ? 0 : 1;
-            if (!lagged && acc != 0.0) ya[in] = fold_add(ya[in], acc, in_wt);
           } else if (lagged) {
             acc = a.pend[lo + i];
+          }
+          if (acc != 0.0) {
+            constexpr int in = M::in_y(0) == M::c_ya(0) ? 0 : 1;
+            if (lagged)
+              in_add = acc * (double)in_wt;
+            else
+              ya[in] = fold_add(ya[in], acc, in_wt);
           }
         }
         if (mem && a.sb.max_rec > 0) rec_k = a.sb.n_rec[i];
@@ -499,8 +510,8 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         cx1 = lagged ? x1_prev : x1;
         need_k1 = true;
         // the loads complete here, not in the loop
-        asm volatile("" ::"v"(ya[0]), "v"(ya[1]), "v"(ref_in), "v"(d.da), "v"(d.db), "v"(in_wt),
-                     "v"(x), "v"(h), "v"(acc), "v"(rec_k), "v"(el));
+        asm volatile("" ::"v"(ya[0]), "v"(ya[1]), "v"(ref_in), "v"(d.da), "v"(d.db), "v"(in_add),
+                     "v"(x), "v"(h), "v"(rec_k), "v"(el));
       }
       d.ra = recip_double(d.da);
       d.rb = recip_double(d.db);
@@ -520,13 +531,35 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       }
       double x_end = cx1 - (double)h_min;
       const int cap = sv.defer_cap();
+      // i for an address that is to be computed where it is used: hoisted out
+      // of the loop such addresses held 24 registers, and the kernel spilled
+      auto here = [](int v) {
+        asm volatile("" : "+v"(v));
+        return v;
+      };
       // The arithmetic runs unmasked in all 64 lanes, groups without a (busy)
       // neuron on harmless values, and only what follows from it is selected
       // by `busy`: a wave whose EXEC mask holds fewer than 16 lanes issues
       // these instructions at a half to a third of the rate (measured: one
       // iteration 1,820 cycles with 16 to 64 lanes on, 4,700-5,800 with 4
       // lanes on in each of a compute unit's four waves).
-      while (__any(busy)) {
+      //
+      // k1 of the next attempt is taken from the new state yn beside the error
+      // ratio and the step factor, before the attempt is accepted: two serial
+      // chains side by side cost little more than one here (8 cycles a
+      // dependent instruction, 4-5 an independent one).  It is taken again
+      // where an event changed the state.
+      auto k1_of = [&](bool sel) {
+        float kn[2];
+        ChainNote nt{ieee ? 0u : ~0u, 0.0f};
+        chain_rhs<M, true>(ya, kn, p, d, mem, nt);
+        if (__any(sel & nt.set())) chain_rhs<M, false>(ya, kn, p, d, mem, nt);
+        k1a[0] = sel ? kn[0] : k1a[0];
+        k1a[1] = sel ? kn[1] : k1a[1];
+      };
+      k1_of(busy);
+      if (__any(busy))
+      for (;;) {
         const bool fresh = busy && need_k1;
         if constexpr (MODE == 2) {
           // learned proposal, as in the loop below; the membrane lanes hold
@@ -549,50 +582,53 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
               h = fminf(h, fmaxf(a.dt * exp2f(o), 2.0f * h_min));
           }
         }
-        unsigned int tiny = ieee ? 0u : ~0u;
-        if (__any(fresh)) {
-          float kn[2];
-          unsigned int tk = ~0u;
-          chain_rhs<M, true>(ya, kn, p, d, mem, tk);
-          tiny = fresh ? min(tiny, tk) : tiny;
+        ChainNote nt{ieee ? 0u : ~0u, 0.0f};
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            k1a[j] = fresh ? kn[j] : k1a[j];
-            ysa[j] = fresh ? fabsf(ya[j]) + fabsf(kn[j] * h) + ck::scal_min : ysa[j];
-          }
-        }
+        for (int j = 0; j < 2; ++j)
+          ysa[j] = fresh ? fabsf(ya[j]) + fabsf(k1a[j] * h) + ck::scal_min : ysa[j];
         const float h_max = (float)(cx1 - x);
         float hh = h;
         if (hh > h_max) hh = h_max;
         if (hh < h_min) hh = h_min;
-        float yn[2];
-        float err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, hh, yn, [&](const float* yy, float* dd) {
-          chain_rhs<M, true>(yy, dd, p, d, mem, tiny);
+        const double xn = x + hh;
+        float yn[2], kn[2];
+        const double rs[2] = {recip_double(ysa[0]), recip_double(ysa[1])};
+        // (a subnormal ratio counts only as the learned form's input; a scale
+        // of inf gives NaN for 0 here, neither of which changes the maximum)
+        auto rel = [&](float v, int j) {
+          if constexpr (MODE == 2) return div_recip(v, rs[j], nt.tiny);
+          return (float)((double)v * rs[j]);
+        };
+        float err = rk5_try<ChainNV>(ckr, ya, k1a, rel, hh, yn, [&](const float* yy, float* dd) {
+          chain_rhs<M, true>(yy, dd, p, d, mem, nt);
         });
+        chain_rhs<M, true>(yn, kn, p, d, mem, nt);
         const float err0 = chain_max<kG>(err);
         err = div_eps(err0);
         bool ok = (err <= 1.0f) | (hh <= h_crit);
         float pw = pow_step_chain(err0, err, ok);
         att_i += busy;
         bool over = false;
-        // rare cases behind one branch: a subnormal quotient (all divisions
-        // again by IEEE), the attempt bound of a non-finite state, an error
-        // ratio outside the range of the fast step factor
+        // What is not an ordinary attempt sits behind one branch.  Rare cases:
+        // a subnormal quotient (all divisions again by IEEE), the attempt
+        // bound of a non-finite state, an error ratio outside the range of
+        // the fast step factor.  Events: ExternalUpdate acts on the membrane,
+        // the step ends or is split.
         const bool need = !ok | (err > ck::err_min);
-        const bool rare = busy & (tiny_noted(tiny) | (att_i > kMaxAttempts) |
+        const bool rare = busy & (nt.set() | (att_i > kMaxAttempts) |
                                   (need & !((err >= kPowLo) & (err <= kPowHi))));
-        if (__builtin_expect(__any(rare), 0)) {
-          if (__any(busy & tiny_noted(tiny))) {
-            float kn[2];
-            chain_rhs<M, false>(ya, kn, p, d, mem, tiny);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              k1a[j] = fresh ? kn[j] : k1a[j];
-              ysa[j] = fresh ? fabsf(ya[j]) + fabsf(kn[j] * h) + ck::scal_min : ysa[j];
-            }
-            err = rk5_try<ChainNV>(ckr, ya, k1a, ysa, hh, yn, [&](const float* yy, float* dd) {
-              chain_rhs<M, false>(yy, dd, p, d, mem, tiny);
+        const bool split = (cap > 0) & !lagged & (att_i >= cap);
+        const bool ext = mem & ((yn[0] < -1.0e3f) | (yn[0] >= p[M::i_thr]) |
+                                (fabsf(yn[1]) > 1.0e6f) | (p[M::i_ref] > 0.0f));
+        const bool event = busy & ok & (ext | (xn >= x_end) | split);
+        const bool other = __any(rare | event);
+        if (__builtin_expect(other, 0) && __any(rare)) {
+          if (__any(busy & nt.set())) {
+            auto rel = [&](float v, int j) { return v / ysa[j]; };
+            err = rk5_try<ChainNV>(ckr, ya, k1a, rel, hh, yn, [&](const float* yy, float* dd) {
+              chain_rhs<M, false>(yy, dd, p, d, mem, nt);
             });
+            chain_rhs<M, false>(yn, kn, p, d, mem, nt);
             err = div_eps(chain_max<kG>(err));
           }
           if (busy & (att_i > kMaxAttempts)) {   // non-finite state: end the step
@@ -611,20 +647,18 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         const float hp = hh * ck::safety * pw;
         const float h_rej = fmaxf(hp, (float)(0.1 * (double)hh));
         const float h_acc = err > ck::err_min ? hp : 5.0f * hh;
-        x = done && !over ? x + hh : x;
+        x = done && !over ? xn : x;
         h = busy ? (ok ? h_acc : h_rej) : h;
-        ya[0] = done ? yn[0] : ya[0];
-        ya[1] = done ? yn[1] : ya[1];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          ya[j] = done ? yn[j] : ya[j];
+          k1a[j] = done ? kn[j] : k1a[j];
+        }
         need_k1 = busy ? ok : need_k1;
         if constexpr (MODE == 2) el = done ? err : el;
-        // events behind one branch: ExternalUpdate acts on the membrane, the
-        // step ends or is split
+        if (!other) continue;
         const bool end_step = x >= x_end;
         const bool m = done & mem;
-        const bool ext = m & ((ya[0] < -1.0e3f) | (ya[0] >= p[M::i_thr]) |
-                              (fabsf(ya[1]) > 1.0e6f) | (p[M::i_ref] > 0.0f));
-        const bool split = (cap > 0) & !lagged & (att_i >= cap);
-        if (!__any(ext | (done & (end_step | split)))) continue;
         const bool off = m && (ya[0] < -1.0e3 || ya[1] < -1.0e6 || ya[1] > 1.0e6);
         const bool refr = m && !off && p[M::i_ref] > 0.0f;
         const bool fire = m && !off && !refr && ya[0] >= p[M::i_thr];
@@ -634,8 +668,9 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         const unsigned long long ms = __ballot(fire);
         if (ms) {
           if (fire) {
-            spike_book(a.sb, a.i0 + i, i, 1.0f, lagged ? t_idx - 1 : t_idx, cx1, &rec_k);
-            const int src = lagged ? (int)((unsigned int)(a.i0 + i) | kSpikeLagBit) : a.i0 + i;
+            const int v = here(i);
+            spike_book(a.sb, a.i0 + v, v, 1.0f, lagged ? t_idx - 1 : t_idx, cx1, &rec_k);
+            const int src = lagged ? (int)((unsigned int)(a.i0 + v) | kSpikeLagBit) : a.i0 + v;
             ya[0] = p[M::i_reset];
             ya[1] += p[M::i_jump];
             const float rr = (float)(int)roundf(p[M::i_tref] / a.dt);
@@ -653,8 +688,8 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         if (__any(resume)) {
           constexpr int in = M::in_y(0) == M::c_ya(0) ? 0 : 1;
           if (resume) {
-            if (port && acc != 0.0) ya[in] = fold_add(ya[in], acc, in_wt);
-            if (mem) a.lag[i] = 0;
+            if (port) ya[in] = (float)((double)ya[in] + in_add);
+            if (mem) a.lag[here(i)] = 0;
             lagged = false;
             cx1 = x1;
             x_end = cx1 - (double)h_min;
@@ -670,13 +705,13 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
             if (ib >= 0) a.var[(size_t)ib * n + i] = ya[1];
             if (mem) {
               if (!end_step) {
-                a.lag[i] = 1;
+                a.lag[here(i)] = 1;
                 ++n_split;
               }
               a.x[i] = x;
               a.h[i] = h;
               if constexpr (MODE == 2) a.err_last[i] = el;
-              if (p[M::i_ref] != ref_in) a.param[(size_t)M::i_ref * n + i] = p[M::i_ref];
+              if (p[M::i_ref] != ref_in) a.param[(size_t)M::i_ref * n + here(i)] = p[M::i_ref];
               hot = !end_step || (p[M::i_ref] <= 0.0f && ya[0] >= M::hot_v(p, a.hot_margin));
               flag_out[i] = hot ? 1 : 0;
             }
@@ -685,11 +720,16 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           const unsigned long long mh = __ballot(hot);
           if (hot) my_hot[hcnt + __popcll(mh & ((1ull << lane) - 1ull))] = i;
           hcnt += __popcll(mh);
+          if (!__any(busy)) break;
         }
+        if (__any(off | refr | fire | resume)) k1_of(done & busy);
       }
       next = end;   // a chain wave takes no share of the bulk
     }
   }
+  double r[M::NPAR];
+#pragma unroll
+  for (int j = 0; j < M::NPAR; ++j) r[j] = UNI && M::divisor(j) ? recip_uniform(p[j]) : 0.0;
   if constexpr (M::NV <= 6 && UNI) {
 #pragma unroll
     for (int j = 0; j < M::NPAR; ++j)
@@ -703,20 +743,18 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
     if (m) {
       if (want) {
         const int v = next + __popcll(m & ((1ull << lane) - 1ull));
-        // (written without a short-circuit on the flag: that form was
-        // compiled with the candidate register overwritten by the flag address)
         int cand = -1;
-        if (v < end) {
-          if (v < n_hw) {
-            cand = dense[hs + v];
-          } else {
-            const int b = b0 + (v - n_hw);
-            const int f = flag_in ? (int)flag_in[b] : 0;
-            cand = f ? -1 : b;
-          }
-        }
+        if (v < end) cand = v < n_hw ? dense[hs + v] : b0 + (v - n_hw);
+        int f = 1;
         if (cand >= 0) {
+          // every load of the neuron that depends on nothing else goes out
+          // together with its hot flag and its ring slots, and a neuron found
+          // on the hot list is dropped afterwards: one round trip to memory
+          // for a refill, where the flag first, then the state, then each
+          // port's slot took three (1e6 AdEx neurons, with the key schedule of
+          // poisson_draw_wave: 67.3 -> 66.0 us a step)
           i = cand;
+          f = flag_in && v >= n_hw ? (int)flag_in[i] : 0;
 #pragma unroll
           for (int j = 0; j < M::NV; ++j) y[j] = a.var[(size_t)j * n + i];
           if (UNI) {
@@ -726,59 +764,68 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
             for (int j = 0; j < M::NPAR; ++j)
               if (a.tab.is_per_neuron(j)) p[j] = a.param[(size_t)j * n + i];
           }
-          ref_in = p[M::i_ref];
           x = a.x[i];
           h = a.h[i];
           if constexpr (MODE != 0) el = a.err_last[i];
           lagged = a.lag ? a.lag[i] != 0 : false;
+          double slot_v[M::NPORT];
+          const long long slot_0 = (long long)sv.pctx().slot * a.pf.n_ch + a.pf.ch_base + i;
           if (sv.prefold()) {
-            // the previous step's fold of this neuron's channels (the fold
-            // kernel's arithmetic): added to the input variables, or kept
-            // as the stashed input of a neuron still inside that step
-            const FoldArgs& f = a.pf;
 #pragma unroll
-            for (int k = 0; k < M::NPORT; ++k) {
-              const long long lo = (long long)k * n;
-              double* rp = f.ring + (size_t)sv.pctx().slot * f.n_ch + (size_t)(f.ch_base + lo + i);
-              double acc = poisson_input(f, lo + i, *rp, sv.pctx().t1, sv.pctx().t_idx,
-                                         f.pu_b < lo + n && f.pu_e > lo);
-              *rp = 0.0;
-              if (lagged) {
-                pend_v[k] = acc;
-              } else if (acc != 0.0) {
-                const int wj = M::in_w(k);
-                const float w = wj >= 0 ? p[wj < 0 ? 0 : wj] : 1.0f;
-                y[M::in_y(k)] = fold_add(y[M::in_y(k)], acc, w);
+            for (int k = 0; k < M::NPORT; ++k) slot_v[k] = a.pf.ring[slot_0 + (long long)k * n];
+          }
+          if (f != 0) i = -1;
+          ref_in = p[M::i_ref];
+          if (f == 0) {
+            if (sv.prefold()) {
+              // the previous step's fold of this neuron's channels (the fold
+              // kernel's arithmetic): added to the input variables, or kept
+              // as the stashed input of a neuron still inside that step
+              const FoldArgs& pf = a.pf;
+#pragma unroll
+              for (int k = 0; k < M::NPORT; ++k) {
+                const long long lo = (long long)k * n;
+                const double acc = poisson_input<true>(pf, lo + i, slot_v[k], sv.pctx().t1,
+                                                       sv.pctx().t_idx,
+                                                       pf.pu_b < lo + n && pf.pu_e > lo);
+                pf.ring[slot_0 + lo] = 0.0;
+                if (lagged) {
+                  pend_v[k] = acc;
+                } else if (acc != 0.0) {
+                  const int wj = M::in_w(k);
+                  const float w = wj >= 0 ? p[wj < 0 ? 0 : wj] : 1.0f;
+                  y[M::in_y(k)] = fold_add(y[M::in_y(k)], acc, w);
+                }
               }
+            } else if (lagged) {
+#pragma unroll
+              for (int k = 0; k < M::NPORT; ++k) pend_v[k] = a.pend[(size_t)k * n + i];
             }
-          } else if (lagged) {
+            if (a.sb.max_rec > 0) rec_k = a.sb.n_rec[i];
+            cx1 = lagged ? x1_prev : x1;
+            need_k1 = true;
+            att_i = 0;
+            // the loads complete here: left pending, the compiler waits for them
+            // where the paths join (the k1 evaluation of every later
+            // iteration), and that wait, counting stores too, would hold the
+            // chain on the stores of finished neurons
 #pragma unroll
-            for (int k = 0; k < M::NPORT; ++k) pend_v[k] = a.pend[(size_t)k * n + i];
+            for (int j = 0; j < M::NV; ++j) asm volatile("" ::"v"(y[j]));
+            if (UNI) {
+              asm volatile("" ::"v"(p[M::i_ref]));
+            } else {
+#pragma unroll
+              for (int j = 0; j < M::NPAR; ++j)
+                if (a.tab.is_per_neuron(j)) asm volatile("" ::"v"(p[j]));
+            }
+            asm volatile("" ::"v"(x), "v"(h));
+            if constexpr (MODE != 0) asm volatile("" ::"v"(el));
+            if (lagged) {
+#pragma unroll
+              for (int k = 0; k < M::NPORT; ++k) asm volatile("" ::"v"(pend_v[k]));
+            }
+            if (a.sb.max_rec > 0) asm volatile("" ::"v"(rec_k));
           }
-          if (a.sb.max_rec > 0) rec_k = a.sb.n_rec[i];
-          cx1 = lagged ? x1_prev : x1;
-          need_k1 = true;
-          att_i = 0;
-          // the loads complete here: left pending, the compiler waits for them
-          // where the paths join (the k1 evaluation of every later
-          // iteration), and that wait, counting stores too, would hold the
-          // chain on the stores of finished neurons
-#pragma unroll
-          for (int j = 0; j < M::NV; ++j) asm volatile("" ::"v"(y[j]));
-          if (UNI) {
-            asm volatile("" ::"v"(p[M::i_ref]));
-          } else {
-#pragma unroll
-            for (int j = 0; j < M::NPAR; ++j)
-              if (a.tab.is_per_neuron(j)) asm volatile("" ::"v"(p[j]));
-          }
-          asm volatile("" ::"v"(x), "v"(h));
-          if constexpr (MODE != 0) asm volatile("" ::"v"(el));
-          if (lagged) {
-#pragma unroll
-            for (int k = 0; k < M::NPORT; ++k) asm volatile("" ::"v"(pend_v[k]));
-          }
-          if (a.sb.max_rec > 0) asm volatile("" ::"v"(rec_k));
         }
       }
       next += __popcll(m);
@@ -830,7 +877,8 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
       }
       if (h < h_min) h = h_min;
       float yn[M::NV];
-      float err = rk5_try<M>(ckr, y, k1, ys, h, yn, [&](const float* yy, float* dd) {
+      auto rel = [&](float v, int j) { return v / ys[j]; };
+      float err = rk5_try<M>(ckr, y, k1, rel, h, yn, [&](const float* yy, float* dd) {
         rhs<M, UNI>(yy, dd, p, r);
       });
       err = div_eps(err);
@@ -1054,15 +1102,15 @@ rk5_persistent_kernel(RK5Args a) {
     __syncthreads();
   }
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = blockIdx.x * (blockDim.x / kWave) +
-                   __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wave = blockIdx.x * (blockDim.x / kWave) + wib;
   const int n_waves = gridDim.x * (blockDim.x / kWave);
   if (a.clear_next_list && blockIdx.x == 0 && threadIdx.x == 0) clear_next_spike_list(a.sl, a.ctx.lst);
   const StepFromArgs sv{a};
   const int n_prev = a.fd.enable ? a.sl.count[a.fd.prev_lst] : 0;
   unsigned long long n_dev = 0;   // synapses delivered by this lane (fused delivery)
-  rk5_persistent_body<M, UNI, MODE>(a, sv, wave, n_waves, wave, s_hot[threadIdx.x / kWave],
-                                    s_spk[threadIdx.x / kWave], &s_pred, n_dev);
+  rk5_persistent_body<M, UNI, MODE>(a, sv, wave, n_waves, wave, s_hot[wib],
+                                    s_spk[wib], &s_pred, n_dev);
   if (a.fd.enable) n_dev += deliver_prev_list(a.fd, a.sl, n_prev, wave, n_waves, lane);
   if (a.ctr) {
     const unsigned int ev = wave_sum32((unsigned int)n_dev);

@@ -6,7 +6,8 @@
 // compiler contracts them; the oracle evaluates the same sequence.
 //
 // Every division of a right-hand side is by a parameter (M::divisor(j)).
-// dv.div(x, p, j) returns x / p[j] (DivIEEE or DivFast, rk5_device.h).
+// dv.div(x, p, j) returns x / p[j], dv.exp_div(x, p, j) exp(x / p[j]) (DivIEEE
+// or DivFast, rk5_device.h).
 // A negated dividend -x/d is written -(x/d) (the same IEEE result) so that
 // x = +0 stays on DivFast's exact path.
 //
@@ -27,7 +28,7 @@
 // c_mem gives the membrane lane's two numerators for the effective potential
 // V from the ports' a (ga(k)), the dividends of parameters c_mv and c_mw (or,
 // where these are -1, dV/dt and dw/dt themselves); c_mx is the divisor of
-// its inner division divx (-1: none).
+// the exponent (-1: none); fx.v(q, V_m) is adex_v, fx.expx(x) exp(x / Delta_T).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -48,15 +49,15 @@ enum AdexTail { aV_th, aDelta_T, ag_L, aE_L, aC_m, aa, ab, atau_w, aI_e, aV_peak
 // (has_i2 false: "- w" follows the product directly and is fused instead).
 // psc: the models that skip the exponential when Delta_T == 0.
 // adex_num: the two numerators (dividends of C_m and tau_w) for the effective
-// potential V; divx(x) is x / Delta_T.
-template <bool PSC, class DX>
+// potential V; fx.expx(x) is exp(x / Delta_T).
+template <bool PSC, class FX>
 __device__ inline void adex_num(const float* q, float V, float w, float i1, float i2, bool has_i1,
-                                bool has_i2, DX&& divx, float* num_v, float* num_w) {
+                                bool has_i2, FX&& fx, float* num_v, float* num_w) {
   float V_spike;
   if (PSC) {
-    V_spike = q[aDelta_T] == 0.0f ? 0.0f : q[aDelta_T] * exp_fma(divx(V - q[aV_th]));
+    V_spike = q[aDelta_T] == 0.0f ? 0.0f : q[aDelta_T] * fx.expx(V - q[aV_th]);
   } else {
-    V_spike = q[aDelta_T] * exp_fma(divx(V - q[aV_th]));
+    V_spike = q[aDelta_T] * fx.expx(V - q[aV_th]);
   }
   float num;
   if (has_i1) {
@@ -76,8 +77,12 @@ __device__ inline void adex_vw(const float* p, float V_m, float w, float i1, flo
   const float* q = p;
   const float V = (q[aref] > 0) ? q[aV_reset] : fminf(V_m, q[aV_peak]);
   float nv, nw;
-  adex_num<PSC>(q, V, w, i1, i2, has_i1, has_i2, [&](float x) { return dv.div(x, q, aDelta_T); },
-                &nv, &nw);
+  struct {
+    D& dv;
+    const float* q;
+    __device__ float expx(float x) { return dv.exp_div(x, q, aDelta_T); }
+  } fx{dv, q};
+  adex_num<PSC>(q, V, w, i1, i2, has_i1, has_i2, fx, &nv, &nw);
   *dV = (q[aref] > 0) ? 0.0f : dv.div(nv, q, aC_m);
   *dw = dv.div(nw, q, atau_w);
 }
@@ -108,14 +113,14 @@ struct AeifCondBeta {
   __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
   __host__ __device__ static constexpr int c_da(int k) { return 14 + 4 * k + 2; }
   __host__ __device__ static constexpr int c_db(int k) { return 14 + 4 * k + 1; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
-    const float V = adex_v(p, V_m);
+    const float V = fx.v(p, V_m);
     float I_syn = 0.0f;
 #pragma unroll
     for (int i = 0; i < NP; ++i) I_syn = fmaf(ga(i), p[14 + 4 * i] - V, I_syn);
-    adex_num<false>(p, V, w, I_syn, 0.0f, true, false, divx, nv, nw);
+    adex_num<false>(p, V, w, I_syn, 0.0f, true, false, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -123,7 +128,7 @@ struct AeifCondBeta {
     const float V = (p[ref] > 0) ? p[V_reset] : fminf(y[0], p[V_peak]);
 #pragma unroll
     for (int i = 0; i < NP; ++i) I_syn = fmaf(y[2 + 2 * i], p[14 + 4 * i] - V, I_syn);
-    const float V_spike = p[Delta_T] * exp_fma(dv.div(V - p[V_th], p, Delta_T));
+    const float V_spike = p[Delta_T] * dv.exp_div(V - p[V_th], p, Delta_T);
     dy[0] = (p[ref] > 0)
                 ? 0.0f
                 : dv.div(fmaf(-p[g_L], V - p[E_L] - V_spike, I_syn) - y[1] + p[I_e], p, C_m);
@@ -157,14 +162,14 @@ struct AeifCondAlpha {
   __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
   __host__ __device__ static constexpr int c_da(int k) { return 14 + 3 * k + 1; }
   __host__ __device__ static constexpr int c_db(int k) { return 14 + 3 * k + 1; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
-    const float V = adex_v(p, V_m);
+    const float V = fx.v(p, V_m);
     float I_syn = 0.0f;
 #pragma unroll
     for (int i = 0; i < NP; ++i) I_syn = fmaf(ga(i), p[14 + 3 * i] - V, I_syn);
-    adex_num<false>(p, V, w, I_syn, 0.0f, true, false, divx, nv, nw);
+    adex_num<false>(p, V, w, I_syn, 0.0f, true, false, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -172,7 +177,7 @@ struct AeifCondAlpha {
     const float V = (p[ref] > 0) ? p[V_reset] : fminf(y[0], p[V_peak]);
 #pragma unroll
     for (int i = 0; i < NP; ++i) I_syn = fmaf(y[2 + 2 * i], p[14 + 3 * i] - V, I_syn);
-    const float V_spike = p[Delta_T] * exp_fma(dv.div(V - p[V_th], p, Delta_T));
+    const float V_spike = p[Delta_T] * dv.exp_div(V - p[V_th], p, Delta_T);
     dy[0] = (p[ref] > 0)
                 ? 0.0f
                 : dv.div(fmaf(-p[g_L], V - p[E_L] - V_spike, I_syn) - y[1] + p[I_e], p, C_m);
@@ -206,13 +211,13 @@ struct AeifPscExp {
   __host__ __device__ static constexpr int c_yb(int) { return -1; }
   __host__ __device__ static constexpr int c_da(int k) { return tau_ex + k; }
   __host__ __device__ static constexpr int c_db(int k) { return tau_ex + k; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m, float w_, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w_, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
     const float* q = p + V_th;
     float I = 0.0f;
     I += ga(0) - ga(1);
-    adex_num<true>(q, adex_v(q, V_m), w_, I, 0.0f, true, false, divx, nv, nw);
+    adex_num<true>(q, fx.v(q, V_m), w_, I, 0.0f, true, false, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -221,7 +226,7 @@ struct AeifPscExp {
     const float V = (p[ref] > 0) ? p[V_reset] : fminf(y[V_m], p[V_peak]);
     const float V_spike = p[Delta_T] == 0.0f
                               ? 0.0f
-                              : p[Delta_T] * exp_fma(dv.div(V - p[V_th], p, Delta_T));
+                              : p[Delta_T] * dv.exp_div(V - p[V_th], p, Delta_T);
     dy[V_m] = (p[ref] > 0)
                   ? 0.0f
                   : dv.div(fmaf(-p[g_L], V - p[E_L] - V_spike, I_syn_tot) - y[w] + p[I_e], p, C_m);
@@ -264,14 +269,14 @@ struct AeifCond2 {
   __host__ __device__ static constexpr int c_yb(int k) { return g1_ex + k; }
   __host__ __device__ static constexpr int c_da(int k) { return tau_d(k); }
   __host__ __device__ static constexpr int c_db(int k) { return tau_r(k); }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m_, float w_, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m_, float w_, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
     const float* q = p + LEAD;
-    const float V = adex_v(q, V_m_);
+    const float V = fx.v(q, V_m_);
     const float I_ex = fmaf(ga(0), p[E_rev_ex] - V, 0.0f);
     const float I_in = fmaf(ga(1), p[E_rev_in] - V, 0.0f);
-    adex_num<false>(q, V, w_, I_ex, I_in, true, true, divx, nv, nw);
+    adex_num<false>(q, V, w_, I_ex, I_in, true, true, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -280,6 +285,7 @@ struct AeifCond2 {
       D& d;
       const float* p;
       __device__ float div(float x, const float*, int j) { return d.div(x, p, LEAD + j); }
+      __device__ float exp_div(float x, const float*, int j) { return d.exp_div(x, p, LEAD + j); }
     } sh{dv, p};
     const float V = adex_v(q, y[V_m]);
     const float I_ex = fmaf(y[g_ex], p[E_rev_ex] - V, 0.0f);
@@ -320,13 +326,13 @@ struct AeifPscAlpha {
   __host__ __device__ static constexpr int c_yb(int k) { return I1_ex + k; }
   __host__ __device__ static constexpr int c_da(int k) { return tau_ex + k; }
   __host__ __device__ static constexpr int c_db(int k) { return tau_ex + k; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m_, float w_, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m_, float w_, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
     const float* q = p + LEAD;
     float I = 0.0f;
     I += ga(0) - ga(1);
-    adex_num<true>(q, adex_v(q, V_m_), w_, I, 0.0f, true, false, divx, nv, nw);
+    adex_num<true>(q, fx.v(q, V_m_), w_, I, 0.0f, true, false, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -335,6 +341,7 @@ struct AeifPscAlpha {
       D& d;
       const float* p;
       __device__ float div(float x, const float*, int j) { return d.div(x, p, LEAD + j); }
+      __device__ float exp_div(float x, const float*, int j) { return d.exp_div(x, p, LEAD + j); }
     } sh{dv, p};
     float I_syn_tot = 0.0f;
     I_syn_tot += y[I_ex] - y[I_in];
@@ -367,13 +374,13 @@ struct AeifPscAlphaMS {
   __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
   __host__ __device__ static constexpr int c_da(int k) { return kAdexTail + 2 * k; }
   __host__ __device__ static constexpr int c_db(int k) { return kAdexTail + 2 * k; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
     float I = 0.0f;
 #pragma unroll
     for (int i = 0; i < NP; ++i) I += ga(i);
-    adex_num<true>(p, adex_v(p, V_m), w, I, 0.0f, true, false, divx, nv, nw);
+    adex_num<true>(p, fx.v(p, V_m), w, I, 0.0f, true, false, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -409,13 +416,13 @@ struct AeifPscExpMS {
   __host__ __device__ static constexpr int c_yb(int) { return -1; }
   __host__ __device__ static constexpr int c_da(int k) { return kAdexTail + k; }
   __host__ __device__ static constexpr int c_db(int k) { return kAdexTail + k; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, DX&& divx,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m, float w, G&& ga, FX&& fx,
                                       float* nv, float* nw) {
     float I = 0.0f;
 #pragma unroll
     for (int i = 0; i < NP; ++i) I += ga(i);
-    adex_num<true>(p, adex_v(p, V_m), w, I, 0.0f, true, false, divx, nv, nw);
+    adex_num<true>(p, fx.v(p, V_m), w, I, 0.0f, true, false, fx, nv, nw);
   }
   template <class D>
   __device__ static inline void deriv(const float* y, float* dy, const float* p, D& dv) {
@@ -465,8 +472,8 @@ struct IzhCondBeta {
   __host__ __device__ static constexpr int c_yb(int k) { return 3 + 2 * k; }
   __host__ __device__ static constexpr int c_da(int k) { return 9 + 4 * k + 2; }
   __host__ __device__ static constexpr int c_db(int k) { return 9 + 4 * k + 1; }
-  template <class G, class DX>
-  __device__ static inline void c_mem(const float* p, float V_m, float u, G&& ga, DX&&, float* dV,
+  template <class G, class FX>
+  __device__ static inline void c_mem(const float* p, float V_m, float u, G&& ga, FX&&, float* dV,
                                       float* du) {
     float I_syn = 0.0f;
     const float V = (p[ref] > 0) ? p[c] : V_m;

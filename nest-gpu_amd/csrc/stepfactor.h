@@ -150,13 +150,12 @@ NGPU_HD inline float div_rn(float a, float d, float r) {
 // fma, and the scaling by 2^k (rounded once where the result is
 // subnormal, overflowing to +inf above ~88.72).  Error < 1 ulp over the
 // whole float range (0.93 ulp at most; 99.5% of results correctly rounded).
-NGPU_HD inline float exp_fma(float x) {
-  // branch-free: the polynomial runs on the clamped argument; at the clamps
-  // the scaling itself overflows (e^100 > 2^128) or underflows to 0 (e^-110 <
-  // 2^-150), and NaN is selected afterwards
-  const float xc = fminf(fmaxf(x, -110.0f), 100.0f);
-  const float k = rintf(xc * 1.44269504f);
-  float r = fmaf(-k, 0.693145752f, xc);
+// ... of |x| <= kExpNear without the clamps: beyond them the scaling overflows
+// or underflows by itself (compared with exp_fma for every such x)
+constexpr float kExpNear = 1.0e6f;
+NGPU_HD inline float exp_fma_near(float x) {
+  const float k = rintf(x * 1.44269504f);
+  float r = fmaf(-k, 0.693145752f, x);
   r = fmaf(-k, 1.42860677e-06f, r);
   float p = 1.0f / 5040.0f;
   p = fmaf(p, r, 1.0f / 720.0f);
@@ -166,7 +165,13 @@ NGPU_HD inline float exp_fma(float x) {
   p = fmaf(p, r, 0.5f);
   p = fmaf(p, r, 1.0f);
   p = fmaf(p, r, 1.0f);
-  const float e = ldexpf(p, (int)k);
+  return ldexpf(p, (int)k);
+}
+NGPU_HD inline float exp_fma(float x) {
+  // branch-free: the polynomial runs on the clamped argument; at the clamps
+  // the scaling itself overflows (e^100 > 2^128) or underflows to 0 (e^-110 <
+  // 2^-150), and NaN is selected afterwards
+  const float e = exp_fma_near(fminf(fmaxf(x, -110.0f), 100.0f));
   return x == x ? e : x;
 }
 
