@@ -305,7 +305,7 @@ class Engine {
   DBuf<uint2> d_pq_;
   int pq_cap_ = 0;
   void build_plastic();
-  void plastic_step(const StepCtx& sc, const SpikeList& sl);
+  StdpArgs stdp_args(const StepCtx& sc, const SpikeList& sl);
   FoldArgs make_fold_args(const Group& g);
   SynTable syn_table() const;
   void fetch_records(long long n_rows);

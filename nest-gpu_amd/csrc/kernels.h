@@ -105,13 +105,13 @@ constexpr int kSynModelStdp = 2;
 constexpr int kSynGroupParams = 8;   // model id, then up to 7 parameters
 constexpr int kMaxSynDt = 16384;     // src/syn_model.h:33
 
-// One step of plastic synapses (after the step's delivery, before the fold
-// of its slot): stdp_arrive_kernel takes the slot's queue -- each event adds
+// One step of plastic synapses: beside the step's delivery
+// (deliver_arrive_kernel) the slot's queue is taken -- each event adds
 // height * weight into the ring, records its arrival step, and depresses
 // the weight if the target fired earlier (src/get_spike.cu:80-95) --, then
-// stdp_post_kernel potentiates the incoming plastic synapses of every
-// neuron that fired this step (src/rev_spike.cu:40-85) and records its
-// spike time.
+// beside the fold of the slot (fold_post_kernel) the incoming plastic synapses
+// of every neuron that fired this step are potentiated (src/rev_spike.cu:40-85)
+// and its spike time is recorded.
 struct StdpArgs {
   SynTable st;
   float* w;                    // = st.syn_w, updated in place
@@ -124,8 +124,8 @@ struct StdpArgs {
   StepCtx ctx;
   SpikeList sl;
   float dt;
+  int blocks;                  // blocks for the step's spikes, at most kDeliverBlocks
 };
-void launch_stdp_step(const StdpArgs& a, hipStream_t s);
 
 // Delivery done by the persistent RK5 kernel (one spike-emitting population)
 // or the batch kernel: its idle waves deliver the previous step's spike list
@@ -417,9 +417,11 @@ void launch_spike_gen(const SpikeGenArgs& a, hipStream_t s);
 void launch_detector(const DetectorArgs& a, hipStream_t s);
 void launch_parrot(const ParrotArgs& a, hipStream_t s);
 void launch_deliver(const DeliverArgs& a, hipStream_t s);   // kDeliverBlocks x 256
+void launch_deliver_arrive(const DeliverArgs& d, const StdpArgs& a, hipStream_t s);
 // the d_int = 0 synapses of the lagged spikes of this step's list (fused delivery)
 void launch_deliver_lagged_d0(const DeliverArgs& a, hipStream_t s);
-void launch_fold(const FoldArgs& a, hipStream_t s);
+// post: the step's post-synaptic updates ride along (null: none)
+void launch_fold(const FoldArgs& a, const StdpArgs* post, hipStream_t s);
 void launch_record(const RecordArgs& a, hipStream_t s);
 
 }  // namespace ngpu
