@@ -1771,7 +1771,7 @@ int Engine::Calibrate() {
   if (const char* env = getenv("NGPU_FUSED_DELIVER")) fused_deliver_env_ = atoi(env) != 0;
   if (const char* env = getenv("NGPU_LAG_D0")) lag_d0_mode_ = atoi(env) == 1 ? 1 : 0;
   if (const char* env = getenv("NGPU_RK5_HOT_LANES")) rk5_hot_lanes_ = std::min(64, std::max(1, atoi(env)));
-  if (const char* env = getenv("NGPU_RK5_CHAIN_WAVES")) rk5_chain_waves_ = std::max(0, atoi(env));
+  if (const char* env = getenv("NGPU_RK5_CHAIN_WAVES")) rk5_chain_waves_ = rk5_chain_waves_learned_ = std::max(0, atoi(env));
   if (const char* env = getenv("NGPU_RK5_LEARNED_CAP")) rk5_learned_cap_ = std::max(0, atoi(env));
   if (const char* env = getenv("NGPU_RK5_DEFER")) {
     rk5_defer_cap_ = std::max(0, atoi(env));
@@ -2035,7 +2035,11 @@ RK5Args Engine::rk5_args(Group& gr, const StepCtx& sc, const SpikeList& sl, cons
     a.hot_margin = rk5_hot_margin_;
     a.hot_only = rk5_hot_only_ ? 1 : 0;
     a.hot_lanes = rk5_hot_lanes_;
-    a.chain_waves = rk5_chain_waves_;
+    // a chain wave takes no share of the bulk, so 1e6 neurons at 3 waves a SIMD
+    // are best with 256 (67.5 us a step; 160 68.0, 320 72.1); with learned
+    // proposals a step has more hot neurons on 2 waves a SIMD (100,000 neurons,
+    // four ports: 256 waves 51.4 us a step, 384 50.8, 512 as 384)
+    a.chain_waves = a.pred_mode == 2 ? rk5_chain_waves_learned_ : rk5_chain_waves_;
   }
   if (g->lag.p) {
     a.lag = g->lag.p;
@@ -2188,6 +2192,9 @@ void Engine::launch_step() {
 // population's fold by its next launch, except after the last step of a
 // Simulate call, where the delivery and fold launches leave the state
 // complete, as without the batch.
+// The launch is made directly: replayed as a one-node graph it leaves a gap of
+// ~8 us between two steps, a direct launch none (the host is ahead by several
+// launches); SetBatchConfig still takes the graph.
 void Engine::plan_batch() {
   batch_on_ = false;
   batch_active_ = false;

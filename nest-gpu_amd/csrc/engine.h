@@ -366,6 +366,7 @@ class Engine {
   bool poisson_runs_ = true;           // uniform poisson connections as runs, not CSR
   int rk5_hot_lanes_ = 32;             // hot entries per wave
   int rk5_chain_waves_ = 256;          // waves the hot entries are spread over in the chain form (0: off)
+  int rk5_chain_waves_learned_ = 384;  // the same with learned step-size proposals
   bool fold_in_rk5_ = true;            // split-step RK5 populations fold inside the next RK5 launch
   bool fused_deliver_env_ = true;      // allow the RK5 launch to deliver the previous step's spikes
   bool fused_deliver_ = false;         // ... and the network qualifies (one emitting RK5 population)
