@@ -237,8 +237,8 @@ int NESTGPU_AMD_Synchronize();
  * Poisson generators is aeif_cond_beta_multisynapse (2 ports),
  * aeif_cond_alpha_multisynapse (4 ports), aeif_psc_exp,
  * izhikevich_cond_beta (2 ports) with uniform parameters, or iaf_psc_exp
- * (2 to 8 populations), each step is one launch, replayed as a one-node HIP
- * graph.  cfg[12] = {on, variant (0: 3 waves per SIMD, 1: 4), iaf_psc_exp
+ * (2 to 8 populations), each step is one launch, made directly or (graph)
+ * replayed as a one-node HIP graph.  cfg[12] = {on, variant (0: 3 waves per SIMD, 1: 4), iaf_psc_exp
  * neurons per lane per pass (1, 2, 4), RK5 block weight x 100, graph,
  * grid blocks, populations, dense (tiled) delivery available, used,
  * channels per tile, tiles, delay rows per tile}.

@@ -2443,7 +2443,7 @@ void Engine::SetBatchConfig(int variant, int iaf_unroll, float rk5_weight, int g
 
 // Autotuner of the batch kernel: register budget (3 or 4 waves per SIMD),
 // iaf_psc_exp unroll (1, 2, 4 neurons per lane per pass), the RK5 block
-// weight (2, 4, 8 per state variable) and, where the network has the tiled
+// weight (1, 2, 4 per state variable) and, where the network has the tiled
 // synapse table, fused delivery or a dense delivery launch, each candidate timed with HIP events
 // around `steps` consecutive steps of the running simulation (a Simulate
 // call of that length); the fastest is kept.  Every candidate computes the
@@ -2459,7 +2459,7 @@ double Engine::AutotuneBatch(int steps, int* n_candidates) {
   for (int t = 0; t <= (tiled_on_ ? 1 : 0); ++t)
     for (int v = 0; v < kBatchVariants; ++v)
       for (int u : {1, 2, 4})
-        for (float w : {2.0f, 4.0f, 8.0f}) cands.push_back({v, u, w, t});
+        for (float w : {1.0f, 2.0f, 4.0f}) cands.push_back({v, u, w, t});
   const float saved_sim = sim_time_;
   const int saved_verb = verbosity_;
   verbosity_ = 0;

@@ -406,7 +406,11 @@ class Engine {
   bool batch_fold_pending_ = false;    // the previous step's fold is left to the next batch launch
   int batch_variant_ = 0;              // register budget: 0 = 3 waves per SIMD, 1 = 4
   int batch_iaf_unroll_ = 0;           // iaf_psc_exp neurons per lane per pass (0: by size, batch_partition)
-  float batch_rk5_weight_ = 4.0f;      // blocks per RK5 neuron and state variable, relative to iaf
+  // blocks per RK5 neuron and state variable, relative to iaf: since hot neurons
+  // are in the chain form a bulk RK5 neuron costs little more than its state
+  // (503,300 neurons of five models: weight 4 201 us a step, 2 118, 1 78, 0.7
+  // 77; 300,000: 124, 76, 61, 61; 50,330 and 840 within 1%)
+  float batch_rk5_weight_ = 1.0f;
   bool batch_graph_on_ = false;        // replay the launch as a HIP graph node (plan_batch says why not)
   int batch_grid_ = 0;
   std::vector<int> batch_groups_;      // group index of each batch population
