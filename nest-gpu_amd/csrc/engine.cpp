@@ -184,6 +184,9 @@ Engine::~Engine() {
     if (r.fp) fclose(r.fp);
   for (auto& p : ev_pending_) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
   for (auto e : ev_free_) (void)hipEventDestroy(e);
+  if (spk_in_flight_) (void)hipEventSynchronize(spk_copied_);
+  if (spk_copied_) (void)hipEventDestroy(spk_copied_);
+  if (spk_copy_) (void)hipHostFree(spk_copy_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -1769,6 +1772,7 @@ int Engine::Calibrate() {
   if (const char* env = getenv("NGPU_POISSON_RUNS")) poisson_runs_ = atoi(env) != 0;
   if (const char* env = getenv("NGPU_FOLD_IN_RK5")) fold_in_rk5_ = atoi(env) != 0;
   if (const char* env = getenv("NGPU_FUSED_DELIVER")) fused_deliver_env_ = atoi(env) != 0;
+  if (const char* env = getenv("NGPU_FUSED_EVENTS")) fused_events_ = std::max(0.0, atof(env));
   if (const char* env = getenv("NGPU_LAG_D0")) lag_d0_mode_ = atoi(env) == 1 ? 1 : 0;
   if (const char* env = getenv("NGPU_RK5_HOT_LANES")) rk5_hot_lanes_ = std::min(64, std::max(1, atoi(env)));
   if (const char* env = getenv("NGPU_RK5_CHAIN_WAVES")) rk5_chain_waves_ = rk5_chain_waves_learned_ = std::max(0, atoi(env));
@@ -2631,22 +2635,57 @@ void Engine::build_tiled(const std::vector<unsigned int>& ch, const std::vector<
 }
 
 // Networks that have the tiled table and whose update launch could deliver
-// the previous step's list itself (fused) choose at the start of each
-// Simulate call by the mean events per step of the call before: up to
-// kFusedEvents the update launch delivers, which saves the 7 us that the
+// the previous step's list itself (fused) choose by the events per step, from
+// the number of spikes delivered in the last kDeliveryCheck steps: up to
+// fused_events_ the update launch delivers, which saves the 7 us that the
 // tiled launch takes for a step with few events (60,000 AdEx neurons with
-// 1,000 synapses, 80,000 events a step: 46 -> 42 us); above, a burst of ten
-// times the mean would cost the update launch's atomics more (1 us per ~23,000
-// events) than the tiles.  The first call, without a mean, is tiled.  The ring
-// receives the same sums either way.
+// 1,000 synapses, 80,000 events a step: 46 -> 42 us); above twice that the
+// tiles do, because the update launch's atomics take 1 us per ~23,000 events
+// and the tiles 1 us per ~60,000; in between it stays as it is.  A network
+// starts tiled.  The count is copied to the host without waiting and looked
+// at a check later, so the choice follows the activity within 64 steps, and
+// the host runs at most 64 steps ahead of the device, far enough to keep it
+// busy.  (Chosen once per Simulate call from the call before, a driven call of
+// 500 steps after a quiet one stayed fused: 100,000 neurons, 4.1e6 events a
+// step, 222 us a step, this way 147.)  The ring receives the same sums either way.
 void Engine::choose_delivery() {
   if (!tiled_on_ || !tiled_auto_ || !(fused_deliver_ || batch_on_)) return;
-  unsigned long long spikes = 0;
-  copy_on(stream_, &spikes, d_stats_.p, sizeof(spikes), hipMemcpyDeviceToHost);
-  if (call_steps_ > 0)
-    tiled_use_ = (double)(spikes - call_spikes_) / (double)call_steps_ * events_per_spike_ > kFusedEvents;
-  call_spikes_ = spikes;
-  call_steps_ = 0;
+  if (steps_run_ - spk_copy_step_ < kDeliveryCheck) return;
+  if (!spk_copied_) {
+    HIPCHK(hipHostMalloc((void**)&spk_copy_, sizeof(*spk_copy_), hipHostMallocDefault));
+    HIPCHK(hipEventCreateWithFlags(&spk_copied_, hipEventDisableTiming));
+  }
+  if (spk_in_flight_) {
+    HIPCHK(hipEventSynchronize(spk_copied_));
+    spk_in_flight_ = false;
+    const double events = (double)(*spk_copy_ - spk_last_) /
+                          (double)(spk_copy_step_ - spk_last_step_) * events_per_spike_;
+    spk_last_ = *spk_copy_;
+    spk_last_step_ = spk_copy_step_;
+    if (events <= fused_events_)
+      set_delivery(false);
+    else if (events > 2.0 * fused_events_)
+      set_delivery(true);
+  }
+  launch_count_out(spk_copy_, d_stats_.p, stream_);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipEventRecord(spk_copied_, stream_));
+  spk_in_flight_ = true;
+  spk_copy_step_ = steps_run_;
+}
+
+// Changes the form of delivery between two steps.
+void Engine::set_delivery(bool tiled) {
+  if (tiled == tiled_use_) return;
+  tiled_use_ = tiled;
+  if (prev_list_pending_) {
+    // fused until now: the list that the next update launch would have
+    // delivered (the d_int = 0 synapses of its lagged spikes are)
+    deliver_list(step_ctx(it_ - 1),
+                 SpikeList{d_spk_count_.p, d_spk_src_.p, d_spk_h_.p, spk_cap_, d_overflow_.p}, 1);
+    prev_list_pending_ = false;
+  }
+  if (batch_active_) batch_upload_args();   // who delivers the lagged spikes' d_int = 0 synapses
 }
 
 // Delivery launch of this step's list: dense (tiled) or global atomics.
@@ -2880,7 +2919,6 @@ int Engine::StartSimulation() {
   // set since the last call, and which populations are recorded decides
   // their split caps)
   // (learned step-size proposals run in the single-population RK5 launches)
-  choose_delivery();
   batch_active_ = batch_on_ && Predictor::get().mode() == 0;
   if (batch_active_) batch_upload_args();
   return 0;
@@ -2895,8 +2933,9 @@ int Engine::SimulationStep() {
     rec_rows_pending_ = 0;
     rec_row_base_ = it_;
   }
+  choose_delivery();
   launch_step();
-  ++call_steps_;
+  ++steps_run_;
   ++rec_rows_pending_;
   long long t_idx = (long long)(int)std::round(neur_t0_ / dt_) + it_ + 1;
   ++it_;

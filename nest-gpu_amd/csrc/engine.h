@@ -380,13 +380,22 @@ class Engine {
   int tiled_env_ = -1;                 // NGPU_TILED: -1 when dense, 0 never, 1 whenever the table fits
   bool tiled_on_ = false;              // the tiled copy of the synapse table exists
   bool tiled_use_ = false;             // deliver with it (a batch autotuner knob)
-  bool tiled_auto_ = false;            // ... chosen per Simulate call (choose_delivery)
+  bool tiled_auto_ = false;            // ... chosen while the network runs (choose_delivery)
   double events_per_spike_ = 0.0;      // mean out-degree of the spiking nodes
   int deliver_parts_log2_ = 0;         // waves that may share a spike's segment (fused delivery)
-  unsigned long long call_spikes_ = 0; // spikes delivered before the last Simulate call
-  long long call_steps_ = 0;           // steps since
-  static constexpr double kFusedEvents = 100000.0;
+  // the choice of delivery: the count of delivered spikes is copied out every
+  // kDeliveryCheck steps and looked at kDeliveryCheck steps later
+  static constexpr int kDeliveryCheck = 32;
+  double fused_events_ = 100000.0;     // events per step up to which delivery is fused (NGPU_FUSED_EVENTS)
+  long long steps_run_ = 0;            // steps since calibration
+  unsigned long long* spk_copy_ = nullptr;   // pinned: the copied count ...
+  hipEvent_t spk_copied_ = nullptr;          // ... there when this has passed
+  bool spk_in_flight_ = false;
+  long long spk_copy_step_ = 0;        // step of the copy
+  unsigned long long spk_last_ = 0;    // the count before, and its step
+  long long spk_last_step_ = 0;
   void choose_delivery();
+  void set_delivery(bool tiled);
   int tile_ch_ = 0, n_tiles_ = 0, tile_rows_ = 0;
   int choose_tile_ch(int rows) const;
   DBuf<uint2> d_toff_;                // (first, end) record of each (source, tile)
