@@ -381,7 +381,7 @@ class Engine {
   bool tiled_on_ = false;              // the tiled copy of the synapse table exists
   bool tiled_use_ = false;             // deliver with it (a batch autotuner knob)
   bool tiled_auto_ = false;            // ... chosen while the network runs (choose_delivery)
-  double events_per_spike_ = 0.0;      // mean out-degree of the spiking nodes
+  double events_per_spike_ = 0.0;      // expected out-degree of a spiking node (Calibrate)
   int deliver_parts_log2_ = 0;         // waves that may share a spike's segment (fused delivery)
   // the choice of delivery: the count of delivered spikes is copied out every
   // kDeliveryCheck steps and looked at kDeliveryCheck steps later

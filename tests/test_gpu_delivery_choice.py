@@ -93,3 +93,28 @@ def test_form_follows_activity(ngpu, monkeypatch, build, defer):
                build, CALLS)
     _same(got, ref)
     assert got[3] == [0, 1, 0, 0, 1]
+
+
+def _hubs(ngpu):
+    # two neurons that hold three quarters of the synapses
+    n = 301
+    p = ngpu.Create("aeif_cond_beta_multisynapse", n, 2)
+    ngpu.SetStatus(p, {"E_rev": [0.0, -85.0], "tau_rise": [1.0, 1.0], "tau_decay": [1.0, 1.0]})
+    hubs = p[0:2]
+    for src, k in ((hubs, 2), (p, 20)):
+        for _ in range(30 if k == 2 else 1):
+            ngpu.Connect(src, p, {"rule": "fixed_indegree", "indegree": k},
+                         {"weight": 0.001, "receptor": 1, "delay": _delay(0.5)})
+    ngpu.SetStatus(hubs, "I_e", 3000.0)
+    return [(p, "V_m")]
+
+
+def test_form_counts_the_hubs(ngpu, monkeypatch):
+    # ~0.04 spikes a step: 300 events a step, 3 by the mean out-degree (80)
+    calls = ((None, 40.0), (None, 40.0))
+    ref = _run(ngpu, monkeypatch, {"NGPU_TILED": "0", "NGPU_FUSED_DELIVER": "0"}, _hubs, calls)
+    n_spk = [len(t) for t in ref[0][0]]
+    assert sum(n_spk[:2]) >= 8 and sum(n_spk[2:]) == 0
+    got = _run(ngpu, monkeypatch, {"NGPU_FUSED_EVENTS": "50"}, _hubs, calls)
+    _same(got, ref)
+    assert got[3] == [1, 1]
