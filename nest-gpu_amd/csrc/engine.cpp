@@ -2427,7 +2427,7 @@ void Engine::batch_step(const StepCtx& sc, const SpikeList& sl) {
 void Engine::GetBatchConfig(int* cfg) {
   cfg[0] = batch_on_ && Predictor::get().mode() == 0 ? 1 : 0;
   cfg[1] = batch_variant_;
-  cfg[2] = batch_iaf_unroll_ > 0 ? batch_iaf_unroll_ : 2;
+  cfg[2] = batch_iaf_unroll_;
   cfg[3] = (int)std::lround(batch_rk5_weight_ * 100.0f);
   cfg[4] = batch_graph_on_ ? 1 : 0;
   cfg[5] = batch_on_ ? batch_grid_ : 0;
@@ -2441,8 +2441,8 @@ void Engine::GetBatchConfig(int* cfg) {
 
 void Engine::SetBatchConfig(int variant, int iaf_unroll, float rk5_weight, int graph, int tiled) {
   if (variant < 0 || variant >= kBatchVariants) throw Error("Batch kernel variant must be 0 or 1");
-  if (iaf_unroll != 1 && iaf_unroll != 2 && iaf_unroll != 4)
-    throw Error("Batch iaf_psc_exp unroll must be 1, 2 or 4");
+  if (iaf_unroll != 0 && iaf_unroll != 1 && iaf_unroll != 2 && iaf_unroll != 4)
+    throw Error("Batch iaf_psc_exp unroll must be 0 (by size), 1, 2 or 4");
   if (!(rk5_weight > 0.0f && rk5_weight < 1.0e6f)) throw Error("Batch RK5 weight must be positive");
   batch_variant_ = variant;
   batch_iaf_unroll_ = iaf_unroll;
@@ -2452,17 +2452,21 @@ void Engine::SetBatchConfig(int variant, int iaf_unroll, float rk5_weight, int g
     if (tiled && !tiled_on_) throw Error("Tiled delivery is not available for this network");
     tiled_use_ = tiled != 0;
     tiled_auto_ = false;
+  } else if (tiled == kTiledAuto) {
+    tiled_auto_ = tiled_on_;
   }
   if (batch_on_) batch_partition();
 }
 
 // Autotuner of the batch kernel: register budget (3 or 4 waves per SIMD),
-// iaf_psc_exp unroll (1, 2, 4 neurons per lane per pass), the RK5 block
+// iaf_psc_exp unroll (by size, 2 or 4 neurons per lane per pass), the RK5 block
 // weight (1, 2, 4 per state variable) and, where the network has the tiled
 // synapse table, fused delivery or a dense delivery launch, each candidate timed with HIP events
 // around `steps` consecutive steps of the running simulation (a Simulate
-// call of that length); the fastest is kept.  Every candidate computes the
-// same results, so tuning on live steps changes nothing but time.
+// call of that length); the fastest is kept (the default configuration is
+// among them).  Where the network chooses its form of delivery by itself, it
+// goes on from the fastest one's.  Every candidate computes the same results,
+// so tuning on live steps changes nothing but time.
 double Engine::AutotuneBatch(int steps, int* n_candidates) {
   if (!calibrated_) Calibrate();
   if (!batch_on_) throw Error("Autotune: the network does not run as one batch launch");
@@ -2473,10 +2477,11 @@ double Engine::AutotuneBatch(int steps, int* n_candidates) {
   std::vector<Cand> cands;
   for (int t = 0; t <= (tiled_on_ ? 1 : 0); ++t)
     for (int v = 0; v < kBatchVariants; ++v)
-      for (int u : {1, 2, 4})
+      for (int u : {0, 2, 4})
         for (float w : {1.0f, 2.0f, 4.0f}) cands.push_back({v, u, w, t});
   const float saved_sim = sim_time_;
   const int saved_verb = verbosity_;
+  const bool automatic = tiled_auto_;
   verbosity_ = 0;
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
@@ -2499,6 +2504,7 @@ double Engine::AutotuneBatch(int steps, int* n_candidates) {
   sim_time_ = saved_sim;
   verbosity_ = saved_verb;
   SetBatchConfig(best.v, best.u, best.w, batch_graph_on_ ? 1 : 0, tiled_on_ ? best.t : -1);
+  tiled_auto_ = automatic;
   if (n_candidates) *n_candidates = (int)cands.size();
   return best_ms / steps;
 }

@@ -265,6 +265,7 @@ class Engine {
   //           delay rows per tile}
   void GetBatchConfig(int* cfg);
   void SetBatchConfig(int variant, int iaf_unroll, float rk5_weight, int graph, int tiled = -1);
+  static constexpr int kTiledAuto = -2;   // SetBatchConfig: the delivery's form chosen by the engine
   double AutotuneBatch(int steps, int* n_candidates);
   void KernelTimes(double* ms, long long* launches);
   void Synchronize();
