@@ -51,8 +51,9 @@ __device__ inline double recip_uniform(float d) {
 // From the hardware's single-precision log2 and exp2 (relative error e of
 // y ~ x^-1/n below 2^-20) one correction in double with the terms to e^2 of
 // (1 - d)^(-1/n), d = 1 - x y^n, leaves an error below 2^-50: correctly
-// rounded for every float in [kPowLo, kPowHi] (exhaustive comparison with
-// pow_m02 / pow_m025 on the device), where those take three Newton steps
+// rounded for every float in [kPowLo, kPowHi] (compared there with pow_m02 /
+// pow_m025, as the other forms here with theirs, by
+// tests/device/arith_check.hip), where those take three Newton steps
 // from a quadratic start, a binade split and a division of the exponent.
 // Outside the range, where a lane needs the value, those are called.
 constexpr float kPowLo = 0x1p-40f, kPowHi = 0x1p100f;

@@ -110,8 +110,6 @@ struct DivFast {
   }
 };
 
-// aeif_cond_beta_multisynapse, src/aeif_cond_beta_multisynapse_kernel.h:165-226
-
 // ---------------------------------------------------------------------------
 // Right-hand side of a population: with uniform divisor parameters (UNI)
 // through DivFast, evaluated again with IEEE divisions when a lane of the

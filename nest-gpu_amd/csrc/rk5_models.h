@@ -8,8 +8,7 @@
 // Every division of a right-hand side is by a parameter (M::divisor(j)).
 // dv.div(x, p, j) returns x / p[j], dv.exp_div(x, p, j) exp(x / p[j]) (DivIEEE
 // or DivFast, rk5_device.h).
-// A negated dividend -x/d is written -(x/d) (the same IEEE result) so that
-// x = +0 stays on DivFast's exact path.
+// A negated dividend -x/d is written -(x/d) (the same IEEE result).
 //
 // Per model: NV state variables, NPAR parameters, NPORT receptor ports;
 // iV/iw the membrane potential and adaptation variable, i_reset/i_thr/

@@ -80,12 +80,10 @@ NGPU_HD inline float pow_m02(float x) {
   return (float)ldexp(z * c5, -q);
 }
 
-// RN(1/d) for a divisor usable by div_rn (normal, |d| in [2^-32, 2^32]),
-// else 0.  1/d rounded to double and then to float is RN(1/d): the exact
-// reciprocal of a float is never within 2^-49 (relative) of a float midpoint.
 // err^-1/5 (five) or err^-1/4 (not five), lane by lane the operations of
-// pow_m02 / pow_m025 with the constants selected: one evaluation serves a
-// wave whose lanes took both the accept and the reject branch.
+// pow_m02 / pow_m025 with the constants selected.  The kernels use
+// pow_step_fast and pow_step_chain (device_common.h), which start from the
+// hardware's log2; this form, of IEEE operations only, is for the host.
 NGPU_HD inline float pow_step(float x, bool five) {
   if (!(x == x)) return x;
   if (x == INFINITY) return 0.0f;
@@ -121,6 +119,9 @@ NGPU_HD inline float pow_step(float x, bool five) {
   return (float)ldexp(z * c, -q);
 }
 
+// RN(1/d) for a divisor usable by div_rn (normal, |d| in [2^-32, 2^32]),
+// else 0.  1/d rounded to double and then to float is RN(1/d): the exact
+// reciprocal of a float is never within 2^-49 (relative) of a float midpoint.
 NGPU_HD inline float recip_rn(float d) {
   const float a = fabsf(d);
   if (!(a >= 0x1p-32f && a <= 0x1p32f)) return 0.0f;
@@ -134,6 +135,7 @@ NGPU_HD inline float recip_rn(float d) {
 // where the quotient or remainder reaches the subnormal range or a is
 // infinite, so dividends outside that range (zeros, subnormals, inf, NaN)
 // take the IEEE division: one integer range test on the magnitude bits.
+// (For the host, as pow_step: the kernels divide by div_recip.)
 NGPU_HD inline float div_rn(float a, float d, float r) {
   unsigned int u;
   __builtin_memcpy(&u, &a, sizeof(u));
@@ -145,13 +147,15 @@ NGPU_HD inline float div_rn(float a, float d, float r) {
 
 // e^x for the exponential term of the AdEx models, in float: Cody-Waite
 // reduction x = k ln2 + r with ln2 split in two floats (the high part has 15
-// significant bits, so k * ln2_hi is exact for the |k| <= 160 reached here),
-// a degree-7 Taylor polynomial of e^r (|r| <= ln2/2) in Horner form with
-// fma, and the scaling by 2^k (rounded once where the result is
-// subnormal, overflowing to +inf above ~88.72).  Error < 1 ulp over the
-// whole float range (0.93 ulp at most; 99.5% of results correctly rounded).
-// ... of |x| <= kExpNear without the clamps: beyond them the scaling overflows
-// or underflows by itself (compared with exp_fma for every such x)
+// significant bits, so k * ln2_hi is exact for the |k| <= 160 that give a
+// finite nonzero result), a degree-7 Taylor polynomial of e^r (|r| <= ln2/2)
+// in Horner form with fma, and the scaling by 2^k (rounded once where the
+// result is subnormal, overflowing to +inf above ~88.72).  Error < 1 ulp over
+// the whole float range (0.93 ulp at most; 99.5% of results correctly
+// rounded).  exp_fma clamps its argument; exp_fma_near is the same for
+// |x| <= kExpNear without the clamps: beyond them k reaches 1.4e6 and r is no
+// longer small, but the scaling overflows or underflows all the same
+// (compared with exp_fma for every such x on the device).
 constexpr float kExpNear = 1.0e6f;
 NGPU_HD inline float exp_fma_near(float x) {
   const float k = rintf(x * 1.44269504f);
