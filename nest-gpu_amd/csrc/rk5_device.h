@@ -451,7 +451,20 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   if constexpr (M::NV <= 6) ckr.hold();
   if constexpr (kChainOk) {
     if (chain && n_hw > 0) {
-      if constexpr (M::NV > 6) ckr.hold();
+      // the chain's tableau in registers; shared with the loop below, as one
+      // set, it cost that loop 24 of them, and from 6 or 7 ports on a kernel
+      // then held one wave per SIMD instead of two (1e6 neurons, 7 ports: 70 Hz
+      // 254 us a step, 178 this way; 460 Hz 670, 435).  Where both ways fit two
+      // waves one set is faster (learned step sizes, 3 ports: 171, 183), and
+      // the Izhikevich models, with more neurons hot at once, are with one
+      // wave (300,000, 7 ports, 280 Hz: 147, 190)
+      constexpr bool kOwn = M::c_mx >= 0 && M::NV > (MODE == 2 ? 10 : UNI ? 12 : 14);
+      CkRegs own;
+      const CkRegs& ckc = kOwn ? own : ckr;
+      if constexpr (kOwn)
+        own.hold();
+      else if constexpr (M::NV > 6)
+        ckr.hold();
       // ---- chain form: one neuron per group of kG lanes (rk5_chain.h) ----
       const int role = lane & (kG - 1), k = role - 1;
       const bool mem = role == 0, port = role >= 1 && role <= M::NPORT;
@@ -597,7 +610,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           if constexpr (MODE == 2) return div_recip(v, rs[j], nt.tiny);
           return (float)((double)v * rs[j]);
         };
-        float err = rk5_try<ChainNV>(ckr, ya, k1a, rel, hh, yn, [&](const float* yy, float* dd) {
+        float err = rk5_try<ChainNV>(ckc, ya, k1a, rel, hh, yn, [&](const float* yy, float* dd) {
           chain_rhs<M, true>(yy, dd, p, d, mem, nt);
         });
         chain_rhs<M, true>(yn, kn, p, d, mem, nt);
@@ -623,7 +636,7 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
         if (__builtin_expect(other, 0) && __any(rare)) {
           if (__any(busy & nt.set())) {
             auto rel = [&](float v, int j) { return v / ysa[j]; };
-            err = rk5_try<ChainNV>(ckr, ya, k1a, rel, hh, yn, [&](const float* yy, float* dd) {
+            err = rk5_try<ChainNV>(ckc, ya, k1a, rel, hh, yn, [&](const float* yy, float* dd) {
               chain_rhs<M, false>(yy, dd, p, d, mem, nt);
             });
             chain_rhs<M, false>(yn, kn, p, d, mem, nt);
