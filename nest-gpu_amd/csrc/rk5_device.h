@@ -422,6 +422,17 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
   double x = 0.0;
   double cx1 = 0.0;     // end of the step the lane's neuron is in (x1, or x1_prev if lagged)
   bool lagged = false;
+  // Models with many ports fold the previous step's slots in a loop that is not
+  // unrolled, over pend_v by selects: unrolled, the loop is too long for the
+  // compiler from 8 ports of two variables on, and its arrays went to scratch
+  // with it (300,000 neurons: izhikevich_cond_beta, 9 ports, 256 us a step, 203
+  // this way; aeif_cond_beta, 12 ports, 446, 354).  With one variable a port
+  // that happens from 17 ports on, where scratch costs less than one wave per
+  // SIMD would (18 ports: 88, 136 this way); from 13 to 16 ports this form
+  // keeps two waves instead of one (16 ports: 108, 81), below it is slower (12
+  // ports: 61, 68).
+  constexpr bool kCompact =
+      M::NPORT > 7 && (M::NV >= 2 + 2 * M::NPORT || (M::NV > 14 && M::NV <= 18));
   // a lagged neuron's stashed input, loaded when the lane takes it, so
   // resuming a split step needs no memory round trip inside the chain
   double pend_v[M::NPORT];
@@ -779,11 +790,11 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
           h = a.h[i];
           if constexpr (MODE != 0) el = a.err_last[i];
           lagged = a.lag ? a.lag[i] != 0 : false;
-          double slot_v[M::NPORT];
+          double slot_v[M::NPORT];   // (kCompact: in pend_v)
           const long long slot_0 = (long long)sv.pctx().slot * a.pf.n_ch + a.pf.ch_base + i;
           if (sv.prefold()) {
 #pragma unroll
-            for (int k = 0; k < M::NPORT; ++k) slot_v[k] = a.pf.ring[slot_0 + (long long)k * n];
+            for (int k = 0; k < M::NPORT; ++k) (kCompact ? pend_v[k] : slot_v[k]) = a.pf.ring[slot_0 + (long long)k * n];
           }
           if (f != 0) i = -1;
           ref_in = p[M::i_ref];
@@ -793,13 +804,28 @@ __device__ __attribute__((always_inline)) inline void rk5_persistent_body(
               // kernel's arithmetic): added to the input variables, or kept
               // as the stashed input of a neuron still inside that step
               const FoldArgs& pf = a.pf;
-#pragma unroll
-              for (int k = 0; k < M::NPORT; ++k) {
+              auto fold = [&](int k, double slot) {
                 const long long lo = (long long)k * n;
-                const double acc = poisson_input<true>(pf, lo + i, slot_v[k], sv.pctx().t1,
+                const double acc = poisson_input<true>(pf, lo + i, slot, sv.pctx().t1,
                                                        sv.pctx().t_idx,
                                                        pf.pu_b < lo + n && pf.pu_e > lo);
                 pf.ring[slot_0 + lo] = 0.0;
+                return acc;
+              };
+              if constexpr (kCompact) {
+#pragma unroll 1
+                for (int k = 0; k < M::NPORT; ++k) {
+                  double v = 0.0;
+#pragma unroll
+                  for (int j = 0; j < M::NPORT; ++j) v = j == k ? pend_v[j] : v;
+                  v = fold(k, v);
+#pragma unroll
+                  for (int j = 0; j < M::NPORT; ++j) pend_v[j] = j == k ? v : pend_v[j];
+                }
+              }
+#pragma unroll
+              for (int k = 0; k < M::NPORT; ++k) {
+                const double acc = kCompact ? pend_v[k] : fold(k, slot_v[k]);
                 if (lagged) {
                   pend_v[k] = acc;
                 } else if (acc != 0.0) {
@@ -1101,9 +1127,13 @@ __device__ inline void clear_next_spike_list(const SpikeList& sl, int lst) {
 // VGPRs, 3 waves per SIMD.  The chain form keeps the tableau and the
 // parameters in vector registers; held to 128 VGPRs (4 waves) it spilled 51
 // of them, and the bulk of a launch runs as fast with 3 waves as with 4.
+// Models of 17 and 18 state variables (8 ports of two each) are held to 256, 2
+// waves: without, some need a few more (300,000 neurons, 8 ports, per-neuron C_m:
+// one wave 274 us a step, two 194).  With 20 and more two waves spill: 300,000
+// neurons, 10 ports, 70 Hz, one wave 223, two 274.
 template <class M, bool UNI, int MODE>
 __global__ void __launch_bounds__(kRK5Block)
-__attribute__((amdgpu_waves_per_eu(M::NV > 6 || MODE == 1 ? 1 : MODE == 2 ? 2 : 3)))
+__attribute__((amdgpu_waves_per_eu(MODE == 1 || M::NV > 18 ? 1 : M::NV > 16 ? 2 : M::NV > 6 ? 1 : MODE == 2 ? 2 : 3)))
 rk5_persistent_kernel(RK5Args a) {
   __shared__ int s_hot[kRK5Block / kWave][kHotLds];
   __shared__ int s_spk[kRK5Block / kWave][kSpkLds];

@@ -1,7 +1,8 @@
 """Registers and scratch memory of the persistent RK5 kernels, from the
 metadata of the built library: what decides how many waves a SIMD holds (512
-registers a lane).  The limits are
-the ones that the kernels' forms were chosen for (rk5_device.h: kOwn)."""
+registers a lane) and whether a neuron's arrays live in memory.  The limits are
+the ones that the kernels' forms were chosen for (rk5_device.h: kOwn, kCompact,
+the register budget)."""
 import os
 import re
 import shutil
@@ -13,8 +14,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "nest-gpu_amd", "libnestgpu_amd.so")
 TOOLS = "/opt/rocm/llvm/bin"
 
-# two variables a port
+# two variables a port / one
 TWO = ("AeifCondBeta", "AeifCondAlpha", "AeifPscAlphaMS", "IzhCondBeta")
+ONE = "AeifPscExpMS"
 
 
 @pytest.fixture(scope="module")
@@ -44,10 +46,23 @@ def kernels(tmp_path_factory):
 
 
 @pytest.mark.parametrize("model", TWO)
-def test_two_waves_up_to_seven_ports(kernels, model):
+def test_two_waves_up_to_eight_ports(kernels, model):
     for (name, ports, uni, mode), (regs, _) in kernels.items():
-        if name == model and ports <= 7 and mode == 0 and (name != "IzhCondBeta" or ports != 7):
+        if name == model and ports <= 8 and mode == 0 and (name != "IzhCondBeta" or ports != 7):
             assert regs <= 256, (ports, uni, regs)
+
+
+@pytest.mark.parametrize("model", TWO)
+def test_no_arrays_in_scratch(kernels, model):
+    # (a few spilled registers are let through)
+    for (name, ports, uni, mode), (_, scratch) in kernels.items():
+        if name == model and mode == 0 and ports <= 17:
+            assert scratch <= 64, (ports, uni, scratch)
+
+
+def test_one_variable_a_port(kernels):
+    for ports in range(1, 17):
+        assert kernels[(ONE, ports, False, 0)][0] <= 256, ports
 
 
 def test_learned_step_sizes_two_waves(kernels):
