@@ -184,8 +184,7 @@ Engine::~Engine() {
     if (r.fp) fclose(r.fp);
   for (auto& p : ev_pending_) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
   for (auto e : ev_free_) (void)hipEventDestroy(e);
-  if (spk_in_flight_) (void)hipEventSynchronize(spk_copied_);
-  if (spk_copied_) (void)hipEventDestroy(spk_copied_);
+  if (spk_in_flight_) (void)hipStreamSynchronize(stream_);
   if (spk_copy_) (void)hipHostFree(spk_copy_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
@@ -2668,12 +2667,20 @@ void Engine::build_tiled(const std::vector<unsigned int>& ch, const std::vector<
 void Engine::choose_delivery() {
   if (!tiled_on_ || !tiled_auto_ || !(fused_deliver_ || batch_on_)) return;
   if (steps_run_ - spk_copy_step_ < kDeliveryCheck) return;
-  if (!spk_copied_) {
-    HIPCHK(hipHostMalloc((void**)&spk_copy_, sizeof(*spk_copy_), hipHostMallocDefault));
-    HIPCHK(hipEventCreateWithFlags(&spk_copied_, hipEventDisableTiming));
+  if (!spk_copy_) {
+    HIPCHK(hipHostMalloc((void**)&spk_copy_, 2 * sizeof(*spk_copy_), hipHostMallocCoherent));
+    spk_copy_[1] = 0;
   }
   if (spk_in_flight_) {
-    HIPCHK(hipEventSynchronize(spk_copied_));
+    // the copy of the check before, for long done unless the device is more
+    // than a check behind; a stream that stops on an error ends the wait
+    for (long long n = 1; __atomic_load_n(&spk_copy_[1], __ATOMIC_ACQUIRE) !=
+                          (unsigned long long)spk_copy_step_; ++n) {
+      if (n % 10000000 == 0)
+        sync_streams();
+      else
+        __builtin_ia32_pause();
+    }
     spk_in_flight_ = false;
     const double events = (double)(*spk_copy_ - spk_last_) /
                           (double)(spk_copy_step_ - spk_last_step_) * events_per_spike_;
@@ -2684,11 +2691,10 @@ void Engine::choose_delivery() {
     else if (events > 2.0 * fused_events_)
       set_delivery(true);
   }
-  launch_count_out(spk_copy_, d_stats_.p, stream_);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipEventRecord(spk_copied_, stream_));
-  spk_in_flight_ = true;
   spk_copy_step_ = steps_run_;
+  launch_count_out(spk_copy_, d_stats_.p, (unsigned long long)spk_copy_step_, stream_);
+  HIPCHK(hipGetLastError());
+  spk_in_flight_ = true;
 }
 
 // Changes the form of delivery between two steps.

@@ -389,10 +389,9 @@ class Engine {
   static constexpr int kDeliveryCheck = 32;
   double fused_events_ = 100000.0;     // events per step up to which delivery is fused (NGPU_FUSED_EVENTS)
   long long steps_run_ = 0;            // steps since calibration
-  unsigned long long* spk_copy_ = nullptr;   // pinned: the copied count ...
-  hipEvent_t spk_copied_ = nullptr;          // ... there when this has passed
+  unsigned long long* spk_copy_ = nullptr;   // pinned: the count, and the step of its copy
   bool spk_in_flight_ = false;
-  long long spk_copy_step_ = 0;        // step of the copy
+  long long spk_copy_step_ = 0;        // step of the last copy
   unsigned long long spk_last_ = 0;    // the count before, and its step
   long long spk_last_step_ = 0;
   void choose_delivery();

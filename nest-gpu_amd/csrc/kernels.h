@@ -417,7 +417,8 @@ void launch_spike_gen(const SpikeGenArgs& a, hipStream_t s);
 void launch_detector(const DetectorArgs& a, hipStream_t s);
 void launch_parrot(const ParrotArgs& a, hipStream_t s);
 void launch_deliver(const DeliverArgs& a, hipStream_t s);   // kDeliverBlocks x 256
-void launch_count_out(unsigned long long* host, const unsigned long long* count, hipStream_t s);
+void launch_count_out(unsigned long long* host, const unsigned long long* count,
+                      unsigned long long tag, hipStream_t s);
 void launch_deliver_arrive(const DeliverArgs& d, const StdpArgs& a, hipStream_t s);
 // the d_int = 0 synapses of the lagged spikes of this step's list (fused delivery)
 void launch_deliver_lagged_d0(const DeliverArgs& a, hipStream_t s);

@@ -238,14 +238,19 @@ void launch_deliver(const DeliverArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(deliver_kernel, dim3(kDeliverBlocks), dim3(256), 0, s, a);
 }
 
-// A count into pinned host memory, between two steps.  Bound: one launch
-// (a copy of the 8 bytes took ~6 us of the stream).
-__global__ void count_out_kernel(unsigned long long* host, const unsigned long long* count) {
-  *host = *count;
+// A count into pinned host memory, between two steps, then its tag, by which
+// the host knows that it is there: host[0], host[1].  Bound: one launch.  A copy
+// of the 8 bytes took ~6 us of the stream, this launch with an event behind
+// it as much (the event's release flushes the caches).
+__global__ void count_out_kernel(unsigned long long* host, const unsigned long long* count,
+                                 unsigned long long tag) {
+  __hip_atomic_store(host, *count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(host + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-void launch_count_out(unsigned long long* host, const unsigned long long* count, hipStream_t s) {
-  hipLaunchKernelGGL(count_out_kernel, dim3(1), dim3(1), 0, s, host, count);
+void launch_count_out(unsigned long long* host, const unsigned long long* count,
+                      unsigned long long tag, hipStream_t s) {
+  hipLaunchKernelGGL(count_out_kernel, dim3(1), dim3(1), 0, s, host, count, tag);
 }
 
 // Dense delivery (TiledDeliverArgs).  The work of a step is a list of items
