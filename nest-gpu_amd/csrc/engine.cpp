@@ -2458,8 +2458,8 @@ void Engine::SetBatchConfig(int variant, int iaf_unroll, float rk5_weight, int g
 }
 
 // Autotuner of the batch kernel: register budget (3 or 4 waves per SIMD),
-// iaf_psc_exp unroll (by size, 2 or 4 neurons per lane per pass), the RK5 block
-// weight (1, 2, 4 per state variable) and, where the network has the tiled
+// iaf_psc_exp unroll (by size, 1, 2 or 4 neurons per lane per pass), the RK5 block
+// weight (1, 2, or, by size only, 4 per state variable) and, where the network has the tiled
 // synapse table, fused delivery or a dense delivery launch, each candidate timed with HIP events
 // around `steps` consecutive steps of the running simulation (a Simulate
 // call of that length); the fastest is kept (the default configuration is
@@ -2476,8 +2476,9 @@ double Engine::AutotuneBatch(int steps, int* n_candidates) {
   std::vector<Cand> cands;
   for (int t = 0; t <= (tiled_on_ ? 1 : 0); ++t)
     for (int v = 0; v < kBatchVariants; ++v)
-      for (int u : {0, 2, 4})
-        for (float w : {1.0f, 2.0f, 4.0f}) cands.push_back({v, u, w, t});
+      for (int u : {0, 1, 2, 4})
+        for (float w : {1.0f, 2.0f, 4.0f})
+          if (w < 4.0f || u == 0) cands.push_back({v, u, w, t});
   const float saved_sim = sim_time_;
   const int saved_verb = verbosity_;
   const bool automatic = tiled_auto_;
